@@ -38,7 +38,8 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch group measured with rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE (fetch scaled x2.000, write x1.000 by a 1 GiB device copy in the
 # same runs); profiles/flcf_c2_hbm_traffic.md has the commands and counts.
-MEASURED_TRAFFIC = {("c2", 16): {"passA": 5.4165e+09, "passB": 8.5902e+09, "passC": 4.9830e+09}}
+# (config, batch) -> pass -> bytes
+MEASURED_TRAFFIC = {}
 
 def log(msg):
     print(msg, file=sys.stderr, flush=True)
@@ -478,6 +479,8 @@ def main():
     roof = None
     if cnt_k[3:6].sum() > 0:
         model = byte_model(cfg, KA)
+        if not cnt_k[4]:  # the y transform runs within the other two
+            del model["passB"]
         dom = max(["passA", "passB", "passC"], key=lambda k: per_kernel[k]["ms_total"])
         i = names.index(dom)
         full = (ntimed // KA) * KA == ntimed

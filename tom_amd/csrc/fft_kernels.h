@@ -141,41 +141,61 @@ class Twiddles {
   ~Twiddles() {
     for (auto& kv : t32_) (void)hipFree(kv.second);
     for (auto& kv : t64_) (void)hipFree(kv.second);
+    for (auto& kv : lists_) (void)hipFree(kv.second);
   }
   const c32* f32(int L) { return get<float>(L, t32_); }
   const c64* f64(int L) { return get<double>(L, t64_); }
 
+  template <typename T>
+  static cpx<T> root(int L, int m) {
+    const double kPi = 3.14159265358979323846264338327950288419716939937510;
+    // exact values at the quarter points keep symmetric inputs symmetric
+    const long q = (long)m * 4;
+    double c, s;
+    if (q % L == 0) {
+      const int k = (int)(q / L) & 3;
+      c = (k == 0) ? 1 : (k == 2) ? -1 : 0;
+      s = (k == 1) ? 1 : (k == 3) ? -1 : 0;
+    } else {
+      c = cos(2 * kPi * m / L);
+      s = sin(2 * kPi * m / L);
+    }
+    return mk<T>((T)c, (T)s);
+  }
+
+  // A list of entries of the f32 tables in an order of its own, made once per
+  // key by make(std::vector<c32>&).
+  template <class F>
+  const c32* list(long key, F&& make) {
+    std::lock_guard<std::mutex> g(mu_);
+    auto it = lists_.find(key);
+    if (it != lists_.end()) return it->second;
+    std::vector<c32> h;
+    make(h);
+    return lists_[key] = upload(h);
+  }
+
  private:
+  template <typename T>
+  static cpx<T>* upload(const std::vector<cpx<T>>& h) {
+    cpx<T>* d = nullptr;
+    TOMHIP_CHECK(hipMalloc(&d, sizeof(cpx<T>) * h.size()));
+    TOMHIP_CHECK(hipMemcpy(d, h.data(), sizeof(cpx<T>) * h.size(), hipMemcpyHostToDevice));
+    return d;
+  }
   template <typename T, typename M>
   const cpx<T>* get(int L, M& map) {
     std::lock_guard<std::mutex> g(mu_);
     auto it = map.find(L);
     if (it != map.end()) return it->second;
     std::vector<cpx<T>> h(L);
-    const double kPi = 3.14159265358979323846264338327950288419716939937510;
-    for (int m = 0; m < L; ++m) {
-      // exact values at the quarter points keep symmetric inputs symmetric
-      const long q = (long)m * 4;
-      double c, s;
-      if (q % L == 0) {
-        const int k = (int)(q / L) & 3;
-        c = (k == 0) ? 1 : (k == 2) ? -1 : 0;
-        s = (k == 1) ? 1 : (k == 3) ? -1 : 0;
-      } else {
-        c = cos(2 * kPi * m / L);
-        s = sin(2 * kPi * m / L);
-      }
-      h[m] = mk<T>((T)c, (T)s);
-    }
-    cpx<T>* d = nullptr;
-    TOMHIP_CHECK(hipMalloc(&d, sizeof(cpx<T>) * L));
-    TOMHIP_CHECK(hipMemcpy(d, h.data(), sizeof(cpx<T>) * L, hipMemcpyHostToDevice));
-    map[L] = d;
-    return d;
+    for (int m = 0; m < L; ++m) h[m] = root<T>(L, m);
+    return map[L] = upload(h);
   }
   std::mutex mu_;
   std::map<int, c32*> t32_;
   std::map<int, c64*> t64_;
+  std::map<long, c32*> lists_;
 };
 
 template <typename T>

@@ -98,6 +98,7 @@ class Search {
   void run_batch(const float* rm_dev, int ka, long first_index, const long* desc);
   void rotate_templates(const float* rm_dev, int count, float* tout, const long* desc, long rm_step);
   void box_filter(int count, float* t, c32* work);
+  bool use_fused(int ka) const;
   void launch_passA(int ka);
   void launch_passB(int ka, int z0, int zn);
   void launch_passC(int ka, int z0, int zn, long first_index, const long* desc);
@@ -143,6 +144,7 @@ class Search {
   c32* Tyn_ = nullptr;       // [KA][nz][Y]
   c32* Tx_ = nullptr;        // [KA][nz][ny][pitch] template x-DFT rows, when they do not fit in Q
   c32* Q_ = nullptr;         // [KA][Z][Y][Xh]
+  c32* Pn_ = nullptr;        // [KA][Z][Y] product at kx = X/2 (fused passes)
   bool started_ = false;
   bool remask_ = true;
   // graph of one full batch, replayed with the device descriptor desc_

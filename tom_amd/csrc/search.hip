@@ -21,6 +21,8 @@
 //             P = F_I conj(F_T), pack P(kx=0) + i P(kx=X/2) into column 0,
 //             z inverse FFT, write Q
 //   passB     per (z, kx tile): y inverse FFT in place
+//             (large batches of the common lengths: passes A to C as two
+//             kernels, fused.hip)
 //   passC     per block of x lines: half-length c2r (pre-twiddle + complex
 //             inverse FFT of X/2) straight into a running per-voxel max and
 //             argmax over the batch's angles, then one compare/update against
@@ -35,7 +37,9 @@
 #include <cmath>
 #include <cstring>
 
+#include "dft16.h"
 #include "fft_io.h"
+#include "fused.h"
 #include "rotate.h"
 #include "search.h"
 
@@ -297,9 +301,10 @@ __global__ __launch_bounds__(NT) void k_tmpl_xdft(const float* t2, c32* Tx, cons
 }
 
 // y: Stockham FFT of the ny template rows placed with the template centre at
-// the origin. grid (Xh/TW, nz, ka). Output Ty[a][uz][ky][kx] for kx < Xh,
-// Tyn[a][uz][ky] for kx = Xh (tile 0 only).
-template <int Y, int TW, int NTT = NT>
+// the origin. grid (Xh/TW, nz, ka). Output Ty[a][uz][ky][kx] for kx < Xh (in
+// the order of fused_ty_index with TILED), Tyn[a][uz][ky] for kx = Xh (tile 0
+// only).
+template <int Y, int TW, int NTT, bool TILED>
 __global__ __launch_bounds__(NTT) void k_tmpl_fwd_y(const c32* Tx, c32* Ty, c32* Tyn, const c32* twYg, int X, int ny,
                                                    int nz) {
   constexpr int P = TW + 1;
@@ -324,11 +329,11 @@ __global__ __launch_bounds__(NTT) void k_tmpl_fwd_y(const c32* Tx, c32* Ty, c32*
     if (uy >= ny) return mk(0.f, 0.f);
     return (c < TW) ? src[(long)uy * XP + c] : srn[(long)uy * XP];
   };
-  c32* dst = Ty + ((long)a * nz + uz) * Y * Xh + tile * TW;
+  c32* dst = Ty + ((long)a * nz + uz) * Y * Xh;
   c32* dn = Tyn + ((long)a * nz + uz) * Y;
   auto st = [&](int, int, int c, int ky, c32 v) {
     if (c < TW)
-      dst[(long)ky * Xh + c] = v;
+      dst[TILED ? fused_ty_index(Y, ky, tile * TW + c) : (long)ky * Xh + tile * TW + c] = v;
     else
       dn[ky] = v;
   };
@@ -462,48 +467,6 @@ __global__ __launch_bounds__(NT_A) void k_passA(const c32* Ty, const c32* Tyn, c
 //     q[z] = sum_k2 W16^-(k2 m2) W256^-(k2 m1) sum_k1 W16^-(k1 m1) P[kz]
 // grid (Xh/TW - 1, Y) for the kx tiles after tile 0 (which carries the
 // Nyquist column and runs k_passA), TW = 16 lines, 256 threads.
-template <int DIR>
-__device__ __forceinline__ c32 w16(int m) {
-  // exp(DIR 2 pi i m / 16) for m in [0, 16)
-  constexpr float c1 = 0.92387953251128675613f, s1 = 0.38268343236508977173f, h = 0.70710678118654752440f;
-  const float cs[5] = {1.f, c1, h, s1, 0.f};  // cos(2 pi m / 16), m = 0..4
-  const int q = m & 3, o = m >> 2;            // m = q + 4 o: rotate by o quarter turns
-  c32 w = mk(cs[q], cs[4 - q]);
-  for (int k = 0; k < o; ++k) w = mk(-w.y, w.x);
-  if (DIR < 0) w.y = -w.y;
-  return w;
-}
-
-template <int DIR>
-__device__ __forceinline__ void dft16(c32* v) {
-  // n = a + 4 b, k = kb + 4 ka: 4-point DFTs over b (in place: (a, kb) at
-  // a + 4 kb), twiddles, 4-point DFTs over a (in place: (kb, ka) at a + 4 kb
-  // with a -> ka), then the register renaming to natural order
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    c32 q[4] = {v[a], v[a + 4], v[a + 8], v[a + 12]};
-    Bfly<float, 4, DIR>::run(q);
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) v[a + 4 * kb] = (a == 0 || kb == 0) ? q[kb] : cmul(q[kb], w16<DIR>(a * kb));
-  }
-#pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
-    c32 q[4] = {v[4 * kb], v[4 * kb + 1], v[4 * kb + 2], v[4 * kb + 3]};
-    Bfly<float, 4, DIR>::run(q);
-#pragma unroll
-    for (int ka = 0; ka < 4; ++ka) v[4 * kb + ka] = q[ka];
-  }
-  // X[kb + 4 ka] sits at v[4 kb + ka]: transpose the 4 x 4 register block
-#pragma unroll
-  for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-    for (int ka = kb + 1; ka < 4; ++ka) {
-      const c32 t = v[4 * kb + ka];
-      v[4 * kb + ka] = v[4 * ka + kb];
-      v[4 * ka + kb] = t;
-    }
-}
-
 // NYQ: the launch for kx tile 0 (grid (1, Y, ka / kNyqApb), kNyqApb
 // orientations per block: its F_I slice is read once per block, and the
 // launch still has Y ka / kNyqApb blocks; 8 measured best of 1, 2, 4, 8),
@@ -1082,6 +1045,7 @@ Search::Search(Twiddles& tw, hipStream_t s, const float* volume, int X_, int Y_,
     TOMHIP_CHECK(hipMalloc(&Ty_, sizeof(c32) * (long)KA_ * nz * Y * Xh));
     TOMHIP_CHECK(hipMalloc(&Tyn_, sizeof(c32) * (long)KA_ * nz * Y));
     TOMHIP_CHECK(hipMalloc(&Q_, sizeof(c32) * (long)KA_ * Z * Y * Xh));
+    if (fused_supported(X, Y, Z, KA_)) TOMHIP_CHECK(hipMalloc(&Pn_, sizeof(c32) * (long)KA_ * Z * Y));
     // the template's x-DFT rows live in Q between the template forward and
     // pass A, unless the template is as large as the volume in y and z
     const long txn = (long)KA_ * nz * ny * tx_pitch(Xh);
@@ -1130,6 +1094,7 @@ void Search::release() {
   (void)hipFree(Tyn_);
   (void)hipFree(Tx_);
   (void)hipFree(Q_);
+  (void)hipFree(Pn_);
   (void)hipFree(mu_);
   (void)hipFree(sig_);
   (void)hipFree(wsh_);
@@ -1141,7 +1106,7 @@ void Search::release() {
   maxc_ = nullptr;
   argm_ = nullptr;
   tmpl_ = t1_ = wsh_ = rm_ = ref_tt_ = nullptr;
-  tbox_ = Ty_ = Tyn_ = Tx_ = Q_ = ref_work_ = nullptr;
+  tbox_ = Ty_ = Tyn_ = Tx_ = Q_ = Pn_ = ref_work_ = nullptr;
   mu_ = sig_ = nullptr;
   mask_ = nullptr;
   drop_graph();
@@ -1355,6 +1320,7 @@ void Search::capture_graph() {
   if (!desc_) TOMHIP_CHECK(hipMalloc(&desc_, sizeof(long) * 2));
   // twiddle tables are allocated on first use, which a capture does not allow
   for (int L : {nx, ny, nz, X, Y, Z, Xh}) (void)tw_.f32(L);
+  if (use_fused(KA_)) fused_prepare(tw_, X, Y, Z);
   hipGraph_t g = nullptr;
   TOMHIP_CHECK(hipStreamBeginCapture(s_, hipStreamCaptureModeThreadLocal));
   try {
@@ -1521,7 +1487,14 @@ void Search::launch_passB(int ka, int z0, int zn) {
   TOMHIP_CHECK(hipGetLastError());
 }
 
+bool Search::use_fused(int ka) const {
+  // The fused kernels take the z transform of 256 as 16 x 16, which is what
+  // 16-wide tiles mean there; a z-chunk asks for the separate passes.
+  return zchunk_ == 0 && (Z != 256 || tile_a_ == 16) && fused_supported(X, Y, Z, ka);
+}
+
 void Search::run_batch(const float* rm_dev, int ka, long first_index, const long* desc) {
+  const bool fused = use_fused(ka);
   timed(K_ROT, [&] { rotate_templates(rm_dev, ka, t1_, desc, 9L * ka); });
   if (wsh_) timed(K_BOX, [&] { box_filter(ka, t1_, tbox_); });
 
@@ -1536,30 +1509,41 @@ void Search::run_batch(const float* rm_dev, int ka, long first_index, const long
       // still lets two blocks share a CU; at Y = 512 one block of 1,024
       // threads per CU on 32-wide tiles measured fastest (0.43 -> 0.36 ms
       // per group of 16 against 16-wide tiles of 256 threads)
+      auto go = [&](auto TWc, auto NTc) {
+        constexpr int TW = decltype(TWc)::value, NTT = decltype(NTc)::value;
+        auto launch = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3(Xh / TW, nz, ka), dim3(NTT), 0, s_, (const c32*)Tx, Ty_, Tyn_, tw_.f32(L), X,
+                             ny, nz);
+        };
+        if (fused)
+          launch(k_tmpl_fwd_y<L, TW, NTT, true>);
+        else
+          launch(k_tmpl_fwd_y<L, TW, NTT, false>);
+      };
+      using std::integral_constant;
       if constexpr (L == 512) {
         if (Xh % 32 == 0)
-          hipLaunchKernelGGL((k_tmpl_fwd_y<L, 32, 1024>), dim3(Xh / 32, nz, ka), dim3(1024), 0, s_, (const c32*)Tx,
-                             Ty_, Tyn_, tw_.f32(L), X, ny, nz);
+          go(integral_constant<int, 32>{}, integral_constant<int, 1024>{});
         else
-          hipLaunchKernelGGL((k_tmpl_fwd_y<L, 16, 512>), dim3(Xh / 16, nz, ka), dim3(512), 0, s_, (const c32*)Tx,
-                             Ty_, Tyn_, tw_.f32(L), X, ny, nz);
+          go(integral_constant<int, 16>{}, integral_constant<int, 512>{});
       } else if constexpr (L >= 1024) {
-        hipLaunchKernelGGL((k_tmpl_fwd_y<L, 8>), dim3(Xh / 8, nz, ka), dim3(NT), 0, s_, (const c32*)Tx, Ty_, Tyn_,
-                           tw_.f32(L), X, ny, nz);
-      } else if constexpr (L >= 512) {
-        hipLaunchKernelGGL((k_tmpl_fwd_y<L, 16>), dim3(Xh / 16, nz, ka), dim3(NT), 0, s_, (const c32*)Tx, Ty_,
-                           Tyn_, tw_.f32(L), X, ny, nz);
+        go(integral_constant<int, 8>{}, integral_constant<int, NT>{});
+      } else if constexpr (L > 512) {
+        go(integral_constant<int, 16>{}, integral_constant<int, NT>{});
       } else {
         if (Xh % 32 == 0)
-          hipLaunchKernelGGL((k_tmpl_fwd_y<L, 32>), dim3(Xh / 32, nz, ka), dim3(NT), 0, s_, (const c32*)Tx, Ty_,
-                             Tyn_, tw_.f32(L), X, ny, nz);
+          go(integral_constant<int, 32>{}, integral_constant<int, NT>{});
         else
-          hipLaunchKernelGGL((k_tmpl_fwd_y<L, 16>), dim3(Xh / 16, nz, ka), dim3(NT), 0, s_, (const c32*)Tx, Ty_,
-                             Tyn_, tw_.f32(L), X, ny, nz);
+          go(integral_constant<int, 16>{}, integral_constant<int, NT>{});
       }
     });
     TOMHIP_CHECK(hipGetLastError());
   });
+  if (fused) {
+    timed(K_PASSA, [&] { fused_a(tw_, s_, Ty_, Tyn_, Pn_, FI_, FIn_, Q_, X, Y, Z, nz, ka); });
+    timed(K_PASSC, [&] { fused_bc(tw_, s_, Q_, maxc_, argm_, X, Y, Z, ka, (int)first_index, desc); });
+    return;
+  }
   timed(K_PASSA, [&] { launch_passA(ka); });
   // passes B and C by z-chunks: a chunk of Q written by B is read back by C
   // while it is still in the memory-side cache
