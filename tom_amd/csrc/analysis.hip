@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "analysis.h"
+#include "pool.h"
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(NTA) void k_renorm_lowstd(const float* T, const flo
 double mean_f64(const double* a, long n, hipStream_t s) {
   const int nb = 512;
   double* part = nullptr;
-  TOMHIP_CHECK(hipMalloc(&part, sizeof(double) * nb));
+  work_get(&part, sizeof(double) * nb, s);
   std::vector<double> h(nb);
   try {
     hipLaunchKernelGGL(k_sum_f64, dim3(nb), dim3(NTA), 0, s, a, n, part);
@@ -183,10 +184,10 @@ double mean_f64(const double* a, long n, hipStream_t s) {
     TOMHIP_CHECK(hipMemcpyAsync(h.data(), part, sizeof(double) * nb, hipMemcpyDeviceToHost, s));
     TOMHIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
-    (void)hipFree(part);
+    work_put(part, s);
     throw;
   }
-  (void)hipFree(part);
+  work_put(part, s);
   double t = 0;
   for (double v : h) t += v;
   return t / (double)n;
@@ -195,7 +196,7 @@ double mean_f64(const double* a, long n, hipStream_t s) {
 double std_f32(const float* a, long n, hipStream_t s) {
   const int nb = 512;
   double* part = nullptr;
-  TOMHIP_CHECK(hipMalloc(&part, sizeof(double) * 2 * nb));
+  work_get(&part, sizeof(double) * 2 * nb, s);
   std::vector<double> h(2 * nb);
   double mean = 0, var = 0;
   try {
@@ -213,10 +214,10 @@ double std_f32(const float* a, long n, hipStream_t s) {
       else var = s2 / (double)n - (s1 / (double)n) * (s1 / (double)n);
     }
   } catch (...) {
-    (void)hipFree(part);
+    work_put(part, s);
     throw;
   }
-  (void)hipFree(part);
+  work_put(part, s);
   return sqrt(var > 0 ? var : 0.0);
 }
 
@@ -257,10 +258,12 @@ void flcf_box(const float* S, int nx, int ny, int nz, const float* tmpl, const f
   TOMHIP_REQUIRE(cnt > 0, ERR_WRONG_INPUT, "mask has no positive voxel");
   int4* doff = nullptr;
   float2* dw = nullptr;
-  TOMHIP_CHECK(hipMalloc(&doff, sizeof(int4) * off.size()));
-  if (hipMalloc(&dw, sizeof(float2) * w.size()) != hipSuccess) {
-    (void)hipFree(doff);
-    TOMHIP_CHECK(hipErrorOutOfMemory);
+  work_get(&doff, sizeof(int4) * off.size(), s);
+  try {
+    work_get(&dw, sizeof(float2) * w.size(), s);
+  } catch (...) {
+    work_put(doff, s);
+    throw;
   }
   try {
     TOMHIP_CHECK(hipMemcpyAsync(doff, off.data(), sizeof(int4) * off.size(), hipMemcpyHostToDevice, s));
@@ -270,12 +273,12 @@ void flcf_box(const float* S, int nx, int ny, int nz, const float* tmpl, const f
     TOMHIP_CHECK(hipGetLastError());
     TOMHIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
-    (void)hipFree(doff);
-    (void)hipFree(dw);
+    work_put(doff, s);
+    work_put(dw, s);
     throw;
   }
-  (void)hipFree(doff);
-  (void)hipFree(dw);
+  work_put(doff, s);
+  work_put(dw, s);
 }
 
 void bestpeak_update(const float* ccc, const float* psr, const float* soc, long n, int rule, int32_t angle,
@@ -287,7 +290,7 @@ void bestpeak_update(const float* ccc, const float* psr, const float* soc, long 
 
 long collect_equal(const float* a, long n, const float* vmax_dev, long cap, long* out_dev, hipStream_t s) {
   unsigned long long* cnt = nullptr;
-  TOMHIP_CHECK(hipMalloc(&cnt, sizeof(unsigned long long)));
+  work_get(&cnt, sizeof(unsigned long long), s);
   unsigned long long h = 0;
   try {
     TOMHIP_CHECK(hipMemsetAsync(cnt, 0, sizeof(unsigned long long), s));
@@ -297,10 +300,10 @@ long collect_equal(const float* a, long n, const float* vmax_dev, long cap, long
     TOMHIP_CHECK(hipMemcpyAsync(&h, cnt, sizeof(h), hipMemcpyDeviceToHost, s));
     TOMHIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
-    (void)hipFree(cnt);
+    work_put(cnt, s);
     throw;
   }
-  (void)hipFree(cnt);
+  work_put(cnt, s);
   return (long)h;
 }
 

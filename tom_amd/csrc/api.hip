@@ -10,6 +10,7 @@
 #include "analysis.h"
 #include "rotate.h"
 #include "picks.h"
+#include "pool.h"
 #include "search.h"
 #include "subtomo.h"
 #include "unet.h"
@@ -80,12 +81,12 @@ class DevBuf {
       host_ = nullptr;
       return;
     }
-    TOMHIP_CHECK(hipMalloc(&dev_, bytes));
+    dev_ = work_get(bytes, s_);
     own_ = true;
     if (in) TOMHIP_CHECK(hipMemcpyAsync(dev_, p, bytes, hipMemcpyHostToDevice, s_));
   }
   ~DevBuf() {
-    if (own_) (void)hipFree(dev_);
+    if (own_) work_put(dev_, s_);
   }
   template <typename T>
   T* get() const { return static_cast<T*>(dev_); }
@@ -143,6 +144,7 @@ int tomhip_init(int device, tomhip_ctx** out) {
     // device address of the allocation-free peak's static scratch, once per device
     peak_scratch_register(device);
     c->tw = std::make_unique<Twiddles>();
+    work_device_up(device);
     *out = c.release();
   });
 }
@@ -153,6 +155,7 @@ void tomhip_destroy(tomhip_ctx* ctx) {
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   ctx->tw.reset();
   if (ctx->own) (void)hipStreamDestroy(ctx->own);
+  work_device_down(ctx->device);
   delete ctx;
 }
 
@@ -188,7 +191,7 @@ int tomhip_rotate3d_f32(tomhip_ctx* ctx, const float* src, float* dst, int64_t n
     for (int d = 0; d < 3 && center; ++d)
       TOMHIP_REQUIRE(std::isfinite(center[d]), ERR_WRONG_INPUT, "center must be finite");
     float* drm = nullptr;
-    TOMHIP_CHECK(hipMalloc(&drm, sizeof(rm)));
+    work_get(&drm, sizeof(rm), s);
     TOMHIP_CHECK(hipMemcpyAsync(drm, rm, sizeof(rm), hipMemcpyHostToDevice, s));
     const float c[3] = {center ? center[0] : (float)((nx + 1) / 2), center ? center[1] : (float)((ny + 1) / 2),
                         center ? center[2] : (float)((nz + 1) / 2)};
@@ -196,7 +199,7 @@ int tomhip_rotate3d_f32(tomhip_ctx* ctx, const float* src, float* dst, int64_t n
                   c[2], 0, s);
     out.commit();
     TOMHIP_CHECK(hipStreamSynchronize(s));
-    (void)hipFree(drm);
+    work_put(drm, s);
   });
 }
 
@@ -241,7 +244,7 @@ int tomhip_rotate3d_batch_f32(tomhip_ctx* ctx, const float* src, float* dst, int
     DevBuf out(s, dst, sizeof(float) * n3 * count, false, true);
     std::vector<float> rm = rotmats(euler, count);
     float* drm = nullptr;
-    TOMHIP_CHECK(hipMalloc(&drm, sizeof(float) * rm.size()));
+    work_get(&drm, sizeof(float) * rm.size(), s);
     TOMHIP_CHECK(hipMemcpyAsync(drm, rm.data(), sizeof(float) * rm.size(), hipMemcpyHostToDevice, s));
     const float c[3] = {center ? center[0] : (float)((nx + 1) / 2), center ? center[1] : (float)((ny + 1) / 2),
                         center ? center[2] : (float)((nz + 1) / 2)};
@@ -249,7 +252,7 @@ int tomhip_rotate3d_batch_f32(tomhip_ctx* ctx, const float* src, float* dst, int
                   (int)ny, (int)nz, c[0], c[1], c[2], n3, s);
     out.commit();
     TOMHIP_CHECK(hipStreamSynchronize(s));
-    (void)hipFree(drm);
+    work_put(drm, s);
   });
 }
 
@@ -360,7 +363,7 @@ static float* shifted_weight(hipStream_t s, const float* Wc, const int64_t* n) {
         o[(z * n[1] + y) * n[0] + x] = h[(sz * n[1] + sy) * n[0] + sx];
       }
   float* d = nullptr;
-  TOMHIP_CHECK(hipMalloc(&d, sizeof(float) * n3));
+  work_get(&d, sizeof(float) * n3, s);
   TOMHIP_CHECK(hipMemcpyAsync(d, o.data(), sizeof(float) * n3, hipMemcpyHostToDevice, s));
   TOMHIP_CHECK(hipStreamSynchronize(s));
   return d;
@@ -383,10 +386,10 @@ int tomhip_prepare_template_f32(tomhip_ctx* ctx, const float* tmpl, const int64_
       prepare_template(*ctx->tw, s, t.get<float>(), (int)n[0], (int)n[1], (int)n[2], m.get<float>(), wsh,
                        o.get<float>(), mu_t, sig_t);
     } catch (...) {
-      (void)hipFree(wsh);
+      work_put(wsh, s);
       throw;
     }
-    (void)hipFree(wsh);
+    work_put(wsh, s);
     o.commit();
     TOMHIP_CHECK(hipStreamSynchronize(s));
   });
@@ -429,10 +432,10 @@ int tomhip_search_set_template(tomhip_search* h, const float* tmpl, const float*
       S.set_template(t.get<float>(), wsh, mu_t, sig_t, remask != 0);
       TOMHIP_CHECK(hipStreamSynchronize(s));
     } catch (...) {
-      (void)hipFree(wsh);
+      work_put(wsh, s);
       throw;
     }
-    (void)hipFree(wsh);
+    work_put(wsh, s);
   });
 }
 
@@ -537,9 +540,9 @@ int tomhip_search_refine(tomhip_search* h, const float* volume, const float* eul
     DevBuf dc(s, c.data(), sizeof(int32_t) * c.size(), true, false);
     float* bs = nullptr;
     int32_t *ba = nullptr, *bp = nullptr;
-    TOMHIP_CHECK(hipMalloc(&bs, sizeof(float) * P));
-    TOMHIP_CHECK(hipMalloc(&ba, sizeof(int32_t) * P));
-    TOMHIP_CHECK(hipMalloc(&bp, sizeof(int32_t) * P));
+    work_get(&bs, sizeof(float) * P, s);
+    work_get(&ba, sizeof(int32_t) * P, s);
+    work_get(&bp, sizeof(int32_t) * P, s);
     std::vector<float> hs(P);
     std::vector<int32_t> ha(P), hp(P);
     try {
@@ -556,14 +559,14 @@ int tomhip_search_refine(tomhip_search* h, const float* volume, const float* eul
       TOMHIP_CHECK(hipMemcpyAsync(hp.data(), bp, sizeof(int32_t) * P, hipMemcpyDeviceToHost, s));
       TOMHIP_CHECK(hipStreamSynchronize(s));
     } catch (...) {
-      (void)hipFree(bs);
-      (void)hipFree(ba);
-      (void)hipFree(bp);
+      work_put(bs, s);
+      work_put(ba, s);
+      work_put(bp, s);
       throw;
     }
-    (void)hipFree(bs);
-    (void)hipFree(ba);
-    (void)hipFree(bp);
+    work_put(bs, s);
+    work_put(ba, s);
+    work_put(bp, s);
     std::vector<int32_t> xyz((size_t)P * 3);
     for (int64_t i = 0; i < P; ++i) {
       const long k = hp[i] < 0 ? 0 : hp[i];
@@ -596,18 +599,18 @@ int tomhip_flcf_search_f32(tomhip_ctx* ctx, const float* volume, const int64_t N
     float* tn = nullptr;
     float* wsh = nullptr;
     auto cleanup = [&] {
-      (void)hipFree(own_mask);
-      (void)hipFree(tn);
-      (void)hipFree(wsh);
+      work_put(own_mask, s);
+      work_put(tn, s);
+      work_put(wsh, s);
     };
     try {
       const float* M = mask ? mk_.get<float>() : nullptr;
       if (!M) {
-        TOMHIP_CHECK(hipMalloc(&own_mask, sizeof(float) * n3));
+        work_get(&own_mask, sizeof(float) * n3, s);
         launch_spheremask_os3((int)n[0], (int)n[1], (int)n[2], own_mask, s);
         M = own_mask;
       }
-      TOMHIP_CHECK(hipMalloc(&tn, sizeof(float) * n3));
+      work_get(&tn, sizeof(float) * n3, s);
       if (W) wsh = shifted_weight(s, w.get<float>(), n);
       double mu_t = 0, sig_t = 1;
       prepare_template(*ctx->tw, s, t.get<float>(), (int)n[0], (int)n[1], (int)n[2], M, wsh, tn, &mu_t, &sig_t);
@@ -645,14 +648,14 @@ int tomhip_os3_corr_f32(tomhip_ctx* ctx, const float* img, const int64_t N[3], c
     int32_t* ang = nullptr;
     float* tren = nullptr;
     auto cleanup = [&] {
-      (void)hipFree(own_mask);
-      (void)hipFree(ang);
-      (void)hipFree(tren);
+      work_put(own_mask, s);
+      work_put(ang, s);
+      work_put(tren, s);
     };
     try {
       const float* M = mask ? mk_.get<float>() : nullptr;
       if (!M) {
-        TOMHIP_CHECK(hipMalloc(&own_mask, sizeof(float) * n3));
+        work_get(&own_mask, sizeof(float) * n3, s);
         launch_spheremask_os3((int)n[0], (int)n[1], (int)n[2], own_mask, s);
         M = own_mask;
       }
@@ -669,7 +672,7 @@ int tomhip_os3_corr_f32(tomhip_ctx* ctx, const float* img, const int64_t N[3], c
       double s_img = 1.0;
       if (mean_f64(S.local_std(), NN, s) < 0.01) {
         s_img = std_f32(v.get<float>(), NN, s);
-        TOMHIP_CHECK(hipMalloc(&tren, sizeof(float) * n3));
+        work_get(&tren, sizeof(float) * n3, s);
         renorm_template_lowstd(t.get<float>(), M, n3, tren, s);
         Tuse = tren;
         hot = !(s_img > 0) || mean_f64(S.local_std(), NN, s) / s_img < 0.01;
@@ -680,7 +683,7 @@ int tomhip_os3_corr_f32(tomhip_ctx* ctx, const float* img, const int64_t N[3], c
       const float zero[3] = {0, 0, 0};
       std::vector<float> rm = rotmats(zero, 1);  // exact identity
       S.run(rm.data(), 1, 0);
-      TOMHIP_CHECK(hipMalloc(&ang, sizeof(int32_t) * NN));
+      work_get(&ang, sizeof(int32_t) * NN, s);
       DevBuf o(s, out, sizeof(float) * NN, false, true);
       S.finalize(o.get<float>(), ang);
       if (hot) zero_where_below(o.get<float>(), S.local_std(), NN, 0.05 * s_img, s);
@@ -710,7 +713,7 @@ int tomhip_flcf_box_f32(tomhip_ctx* ctx, const float* search, const float* tmpl,
     try {
       const float* M = mask ? mk_.get<float>() : nullptr;
       if (!M) {  // tom_os3_corr's default: tom_os3_sphereMask(template)
-        TOMHIP_CHECK(hipMalloc(&own_mask, sizeof(float) * n3));
+        work_get(&own_mask, sizeof(float) * n3, s);
         launch_spheremask_os3((int)n[0], (int)n[1], (int)n[2], own_mask, s);
         M = own_mask;
       }
@@ -720,10 +723,10 @@ int tomhip_flcf_box_f32(tomhip_ctx* ctx, const float* search, const float* tmpl,
       o.commit();
       TOMHIP_CHECK(hipStreamSynchronize(s));
     } catch (...) {
-      (void)hipFree(own_mask);
+      work_put(own_mask, s);
       throw;
     }
-    (void)hipFree(own_mask);
+    work_put(own_mask, s);
   });
 }
 
@@ -774,20 +777,20 @@ int tomhip_peak_all_f32(tomhip_ctx* ctx, const float* map, const int64_t N[3], f
     long k = 0;
     std::vector<long> h;
     try {
-      TOMHIP_CHECK(hipMalloc(&dv, sizeof(float)));
-      TOMHIP_CHECK(hipMalloc(&idx, sizeof(long) * capacity));
+      work_get(&dv, sizeof(float), s);
+      work_get(&idx, sizeof(long) * capacity, s);
       TOMHIP_CHECK(hipMemcpyAsync(dv, &v, sizeof(float), hipMemcpyHostToDevice, s));
       k = collect_equal(in.get<float>(), NN, dv, capacity, idx, s);
       h.resize((size_t)std::min<long>(k, capacity));
       TOMHIP_CHECK(hipMemcpyAsync(h.data(), idx, sizeof(long) * h.size(), hipMemcpyDeviceToHost, s));
       TOMHIP_CHECK(hipStreamSynchronize(s));
     } catch (...) {
-      (void)hipFree(dv);
-      (void)hipFree(idx);
+      work_put(dv, s);
+      work_put(idx, s);
       throw;
     }
-    (void)hipFree(dv);
-    (void)hipFree(idx);
+    work_put(dv, s);
+    work_put(idx, s);
     TOMHIP_REQUIRE(k <= capacity, ERR_WRONG_INPUT,
                    std::to_string(k) + " tied maxima exceed the capacity " + std::to_string(capacity));
     std::sort(h.begin(), h.end());  // MATLAB's find order: x fastest
@@ -935,13 +938,13 @@ int tomhip_bin_f32(tomhip_ctx* ctx, const float* in, const int64_t N[3], int nbi
       // ping-pong buffers sized by the first two outputs (later ones shrink)
       float* tmp[2] = {nullptr, nullptr};
       auto release = [&] {
-        (void)hipFree(tmp[0]);
-        (void)hipFree(tmp[1]);
+        work_put(tmp[0], s);
+        work_put(tmp[1], s);
       };
       try {
         long x = N[0], y = N[1], z = N[2];
-        if (nbin > 1) TOMHIP_CHECK(hipMalloc(&tmp[0], sizeof(float) * (x / 2) * (y / 2) * (z / 2)));
-        if (nbin > 2) TOMHIP_CHECK(hipMalloc(&tmp[1], sizeof(float) * (x / 4) * (y / 4) * (z / 4)));
+        if (nbin > 1) work_get(&tmp[0], sizeof(float) * (x / 2) * (y / 2) * (z / 2), s);
+        if (nbin > 2) work_get(&tmp[1], sizeof(float) * (x / 4) * (y / 4) * (z / 4), s);
         const float* src = v.get<float>();
         for (int i = 0; i < nbin; ++i) {
           float* dst = (i == nbin - 1) ? o.get<float>() : tmp[i & 1];
@@ -973,14 +976,14 @@ int tomhip_psr_f32(tomhip_ctx* ctx, const float* xcf, const int64_t N[3], const 
     float* ring = nullptr;
     double *mu = nullptr, *sig = nullptr;
     auto release = [&] {
-      (void)hipFree(ring);
-      (void)hipFree(mu);
-      (void)hipFree(sig);
+      work_put(ring, s);
+      work_put(mu, s);
+      work_put(sig, s);
     };
     try {
-      TOMHIP_CHECK(hipMalloc(&ring, sizeof(float) * n3));
-      TOMHIP_CHECK(hipMalloc(&mu, sizeof(double) * NN));
-      TOMHIP_CHECK(hipMalloc(&sig, sizeof(double) * NN));
+      work_get(&ring, sizeof(float) * n3, s);
+      work_get(&mu, sizeof(double) * NN, s);
+      work_get(&sig, sizeof(double) * NN, s);
       launch_psr_ring((int)n[0], (int)n[1], (int)n[2], ring, s);
       local_stats(*ctx->tw, s, x.get<float>(), (int)N[0], (int)N[1], (int)N[2], ring, (int)n[0], (int)n[1],
                   (int)n[2], mu, sig);
@@ -1137,7 +1140,7 @@ int tomhip_subtomo_score_batch(tomhip_ctx* ctx, int nbox, const int32_t* box_edg
     std::vector<void*> tmp;
     auto up = [&](const void* h, size_t bytes) {
       void* d = nullptr;
-      TOMHIP_CHECK(hipMalloc(&d, bytes));
+      work_get(&d, bytes, s);
       tmp.push_back(d);
       TOMHIP_CHECK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
       return d;
@@ -1154,10 +1157,10 @@ int tomhip_subtomo_score_batch(tomhip_ctx* ctx, int nbox, const int32_t* box_edg
       oC.commit();
       TOMHIP_CHECK(hipStreamSynchronize(s));
     } catch (...) {
-      for (void* p : tmp) (void)hipFree(p);
+      for (void* p : tmp) work_put(p, s);
       throw;
     }
-    for (void* p : tmp) (void)hipFree(p);
+    for (void* p : tmp) work_put(p, s);
   });
 }
 

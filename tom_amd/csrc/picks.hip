@@ -20,6 +20,7 @@
 
 #include "common.h"
 #include "picks.h"
+#include "pool.h"
 
 namespace tomhip {
 
@@ -612,21 +613,21 @@ long picklist(const float* map, int X, int Y, int Z, const int32_t* angles, int 
   long* cnt = nullptr;
   long count = 0;
   auto release = [&] {
-    (void)hipFree(work);
-    (void)hipFree(br);
-    (void)hipFree(sup);
-    (void)hipFree(bad);
-    (void)hipFree(tmp);
-    (void)hipFree(cnt);
+    work_put(work, s);
+    work_put(br, s);
+    work_put(sup, s);
+    work_put(bad, s);
+    work_put(tmp, s);
+    work_put(cnt, s);
   };
   if (n <= 0) return 0;
   try {
-    TOMHIP_CHECK(hipMalloc(&work, sizeof(float) * BV * NB));
-    TOMHIP_CHECK(hipMalloc(&br, sizeof(Brick) * NB));
-    TOMHIP_CHECK(hipMalloc(&sup, sizeof(Brick) * NS));
-    TOMHIP_CHECK(hipMalloc(&bad, sizeof(int)));
-    TOMHIP_CHECK(hipMalloc(&tmp, sizeof(float) * box));
-    TOMHIP_CHECK(hipMalloc(&cnt, sizeof(long)));
+    work_get(&work, sizeof(float) * BV * NB, s);
+    work_get(&br, sizeof(Brick) * NB, s);
+    work_get(&sup, sizeof(Brick) * NS, s);
+    work_get(&bad, sizeof(int), s);
+    work_get(&tmp, sizeof(float) * box, s);
+    work_get(&cnt, sizeof(long), s);
     unsigned g = (unsigned)((N + NTP - 1) / NTP);
     if (g > 16384) g = 16384;
     hipLaunchKernelGGL(k_to_bricks, dim3(g), dim3(NTP), 0, s, map, work, X, Y, Z, NBX, NBY, (int)border,
@@ -651,7 +652,7 @@ long picklist(const float* map, int X, int Y, int Z, const int32_t* angles, int 
 
 long local_maxima(const float* map, int X, int Y, int Z, int r, float thr, long cap, float* out, hipStream_t s) {
   unsigned long long* counter = nullptr;
-  TOMHIP_CHECK(hipMalloc(&counter, sizeof(unsigned long long)));
+  work_get(&counter, sizeof(unsigned long long), s);
   unsigned long long total = 0;
   try {
     TOMHIP_CHECK(hipMemsetAsync(counter, 0, sizeof(unsigned long long), s));
@@ -664,10 +665,10 @@ long local_maxima(const float* map, int X, int Y, int Z, int r, float thr, long 
     TOMHIP_CHECK(hipMemcpyAsync(&total, counter, sizeof(total), hipMemcpyDeviceToHost, s));
     TOMHIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
-    (void)hipFree(counter);
+    work_put(counter, s);
     throw;
   }
-  (void)hipFree(counter);
+  work_put(counter, s);
   return (long)total;
 }
 

@@ -1,0 +1,25 @@
+// Device workspaces of the calls, kept between calls.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+
+namespace tomhip {
+
+// A device workspace of at least `bytes` on the current device, for work on
+// stream s (throws like TOMHIP_CHECK(hipMalloc)).
+void* work_get(size_t bytes, hipStream_t s);
+template <typename T>
+void work_get(T** p, size_t bytes, hipStream_t s) {
+  *p = static_cast<T*>(work_get(bytes, s));
+}
+// Gives a workspace back; what is queued on s so far may still use it. Null
+// is ignored.
+void work_put(const void* p, hipStream_t s) noexcept;
+// The same for a workspace that nothing queued anywhere uses.
+void work_put_idle(const void* p) noexcept;
+
+// Contexts of a device, counted: the last one to go frees what is kept.
+void work_device_up(int device);
+void work_device_down(int device) noexcept;
+
+}  // namespace tomhip

@@ -40,6 +40,7 @@
 #include "dft16.h"
 #include "fft_io.h"
 #include "fused.h"
+#include "pool.h"
 #include "rotate.h"
 #include "search.h"
 
@@ -1034,27 +1035,27 @@ Search::Search(Twiddles& tw, hipStream_t s, const float* volume, int X_, int Y_,
     mask_sum_ = msum;
   }
   try {
-    TOMHIP_CHECK(hipMalloc(&FI_, sizeof(c32) * (long)Z * Y * Xh));
-    TOMHIP_CHECK(hipMalloc(&FIn_, sizeof(c32) * (long)Y * Z));
-    TOMHIP_CHECK(hipMalloc(&maxc_, sizeof(float) * N));
-    TOMHIP_CHECK(hipMalloc(&argm_, sizeof(int32_t) * N));
-    TOMHIP_CHECK(hipMalloc(&tmpl_, sizeof(float) * n3));
-    TOMHIP_CHECK(hipMalloc(&tpairs_, sizeof(float2) * n3));
-    TOMHIP_CHECK(hipMalloc(&t1_, sizeof(float) * n3 * KA_));
-    TOMHIP_CHECK(hipMalloc(&tbox_, sizeof(c32) * n3 * KA_));
-    TOMHIP_CHECK(hipMalloc(&Ty_, sizeof(c32) * (long)KA_ * nz * Y * Xh));
-    TOMHIP_CHECK(hipMalloc(&Tyn_, sizeof(c32) * (long)KA_ * nz * Y));
-    TOMHIP_CHECK(hipMalloc(&Q_, sizeof(c32) * (long)KA_ * Z * Y * Xh));
-    if (fused_supported(X, Y, Z, KA_)) TOMHIP_CHECK(hipMalloc(&Pn_, sizeof(c32) * (long)KA_ * Z * Y));
+    work_get(&FI_, sizeof(c32) * (long)Z * Y * Xh, s_);
+    work_get(&FIn_, sizeof(c32) * (long)Y * Z, s_);
+    work_get(&maxc_, sizeof(float) * N, s_);
+    work_get(&argm_, sizeof(int32_t) * N, s_);
+    work_get(&tmpl_, sizeof(float) * n3, s_);
+    work_get(&tpairs_, sizeof(float2) * n3, s_);
+    work_get(&t1_, sizeof(float) * n3 * KA_, s_);
+    work_get(&tbox_, sizeof(c32) * n3 * KA_, s_);
+    work_get(&Ty_, sizeof(c32) * (long)KA_ * nz * Y * Xh, s_);
+    work_get(&Tyn_, sizeof(c32) * (long)KA_ * nz * Y, s_);
+    work_get(&Q_, sizeof(c32) * (long)KA_ * Z * Y * Xh, s_);
+    if (fused_supported(X, Y, Z, KA_)) work_get(&Pn_, sizeof(c32) * (long)KA_ * Z * Y, s_);
     // the template's x-DFT rows live in Q between the template forward and
     // pass A, unless the template is as large as the volume in y and z
     const long txn = (long)KA_ * nz * ny * tx_pitch(Xh);
-    if (txn > (long)KA_ * Z * Y * Xh) TOMHIP_CHECK(hipMalloc(&Tx_, sizeof(c32) * txn));
+    if (txn > (long)KA_ * Z * Y * Xh) work_get(&Tx_, sizeof(c32) * txn, s_);
     if (mode == MODE_FLCF) {
-      TOMHIP_CHECK(hipMalloc(&mu_, sizeof(double) * N));
-      TOMHIP_CHECK(hipMalloc(&sig_, sizeof(double) * N));
+      work_get(&mu_, sizeof(double) * N, s_);
+      work_get(&sig_, sizeof(double) * N, s_);
       float* mk_ = nullptr;
-      TOMHIP_CHECK(hipMalloc(&mk_, sizeof(float) * n3 * 2));
+      work_get(&mk_, sizeof(float) * n3 * 2, s_);
       mask_ = mk_;
       TOMHIP_CHECK(hipMemcpyAsync(mk_, mask, sizeof(float) * n3, hipMemcpyDeviceToDevice, s_));
       hipLaunchKernelGGL(k_square, dim3(grid_for(n3)), dim3(NT), 0, s_, mk_, mk_ + n3, n3);
@@ -1081,27 +1082,30 @@ void Search::bind_stream(hipStream_t s) {
 Search::~Search() { release(); }
 
 void Search::release() {
-  (void)hipFree(FI_);
-  (void)hipFree(FIn_);
-  (void)hipFree(maxc_);
-  (void)hipFree(argm_);
-  (void)hipFree(tmpl_);
-  (void)hipFree(tpairs_);
+  // whatever stream the plan last ran on may be gone by now: all work is done
+  // before its buffers are given back
+  (void)hipDeviceSynchronize();
+  work_put_idle(FI_);
+  work_put_idle(FIn_);
+  work_put_idle(maxc_);
+  work_put_idle(argm_);
+  work_put_idle(tmpl_);
+  work_put_idle(tpairs_);
   tpairs_ = nullptr;
-  (void)hipFree(t1_);
-  (void)hipFree(tbox_);
-  (void)hipFree(Ty_);
-  (void)hipFree(Tyn_);
-  (void)hipFree(Tx_);
-  (void)hipFree(Q_);
-  (void)hipFree(Pn_);
-  (void)hipFree(mu_);
-  (void)hipFree(sig_);
-  (void)hipFree(wsh_);
-  (void)hipFree(rm_);
-  (void)hipFree(ref_tt_);
-  (void)hipFree(ref_work_);
-  (void)hipFree(const_cast<float*>(mask_));
+  work_put_idle(t1_);
+  work_put_idle(tbox_);
+  work_put_idle(Ty_);
+  work_put_idle(Tyn_);
+  work_put_idle(Tx_);
+  work_put_idle(Q_);
+  work_put_idle(Pn_);
+  work_put_idle(mu_);
+  work_put_idle(sig_);
+  work_put_idle(wsh_);
+  work_put_idle(rm_);
+  work_put_idle(ref_tt_);
+  work_put_idle(ref_work_);
+  work_put_idle(const_cast<float*>(mask_));
   FI_ = FIn_ = nullptr;
   maxc_ = nullptr;
   argm_ = nullptr;
@@ -1110,7 +1114,7 @@ void Search::release() {
   mu_ = sig_ = nullptr;
   mask_ = nullptr;
   drop_graph();
-  (void)hipFree(desc_);
+  work_put_idle(desc_);
   desc_ = nullptr;
   for (auto& e : evpool_) {
     (void)hipEventDestroy(e.a);
@@ -1127,7 +1131,7 @@ namespace {
 void global_moments(const float* volume, long N, hipStream_t s, double* g_out, double* var_out) {
   const int nb = 1024;
   double* part = nullptr;
-  TOMHIP_CHECK(hipMalloc(&part, sizeof(double) * nb));
+  work_get(&part, sizeof(double) * nb, s);
   std::vector<double> hp(nb);
   try {
     hipLaunchKernelGGL(k_partial_sum, dim3(nb), dim3(NT), 0, s, volume, N, 0.0, 0, part);
@@ -1144,10 +1148,10 @@ void global_moments(const float* volume, long N, hipStream_t s, double* g_out, d
     *g_out = g;
     *var_out = ss / (double)N;
   } catch (...) {
-    (void)hipFree(part);
+    work_put(part, s);
     throw;
   }
-  (void)hipFree(part);
+  work_put(part, s);
 }
 
 // Local mean / std under the mask from A = FFT((V-g) + i (V-g)^2) (FP64;
@@ -1156,7 +1160,7 @@ void stats_from_spectrum(c64* A, Twiddles& tw, hipStream_t s, int X, int Y, int 
                          int ny, int nz, double m, double mask_sum, double g, double varg, double* mu, double* sig) {
   const long N = (long)X * Y * Z;
   c64* B = nullptr;
-  TOMHIP_CHECK(hipMalloc(&B, sizeof(c64) * N));
+  work_get(&B, sizeof(c64) * N, s);
   try {
     hipLaunchKernelGGL(k_place_mask, dim3(grid_for(N)), dim3(NT), 0, s, mask, nx, ny, nz, X, Y, Z, B);
     TOMHIP_CHECK(hipGetLastError());
@@ -1170,10 +1174,10 @@ void stats_from_spectrum(c64* A, Twiddles& tw, hipStream_t s, int X, int Y, int 
     TOMHIP_CHECK(hipGetLastError());
     TOMHIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
-    (void)hipFree(B);
+    work_put(B, s);
     throw;
   }
-  (void)hipFree(B);
+  work_put(B, s);
 }
 
 }  // namespace
@@ -1196,24 +1200,24 @@ void local_stats(Twiddles& tw, hipStream_t s, const float* volume, int X, int Y,
   double g, varg;
   global_moments(volume, N, s, &g, &varg);
   c64* A = nullptr;
-  TOMHIP_CHECK(hipMalloc(&A, sizeof(c64) * N));
+  work_get(&A, sizeof(c64) * N, s);
   try {
     hipLaunchKernelGGL(k_make_c, dim3(grid_for(N)), dim3(NT), 0, s, volume, N, g, A);
     TOMHIP_CHECK(hipGetLastError());
     fft3_c2c<double>(A, X, Y, Z, 1, -1, tw, s);
     stats_from_spectrum(A, tw, s, X, Y, Z, mask, nx, ny, nz, m, msum, g, varg, mu, sig);
   } catch (...) {
-    (void)hipFree(A);
+    work_put(A, s);
     throw;
   }
-  (void)hipFree(A);
+  work_put(A, s);
 }
 
 void Search::precompute_stats(const float* volume) {
   double g, varg;
   global_moments(volume, N, s_, &g, &varg);
   c64* A = nullptr;
-  TOMHIP_CHECK(hipMalloc(&A, sizeof(c64) * N));
+  work_get(&A, sizeof(c64) * N, s_);
   try {
     hipLaunchKernelGGL(k_make_c, dim3(grid_for(N)), dim3(NT), 0, s_, volume, N, g, A);
     TOMHIP_CHECK(hipGetLastError());
@@ -1224,10 +1228,10 @@ void Search::precompute_stats(const float* volume) {
     if (mode == MODE_FLCF) stats_from_spectrum(A, tw_, s_, X, Y, Z, mask_, nx, ny, nz, m, mask_sum_, g, varg, mu_, sig_);
     TOMHIP_CHECK(hipStreamSynchronize(s_));
   } catch (...) {
-    (void)hipFree(A);
+    work_put(A, s_);
     throw;
   }
-  (void)hipFree(A);
+  work_put(A, s_);
 }
 
 void Search::set_template(const float* tmpl, const float* wsh, double mu_t_, double sig_t_, bool remask) {
@@ -1240,12 +1244,12 @@ void Search::set_template(const float* tmpl, const float* wsh, double mu_t_, dou
     TOMHIP_REQUIRE(supported_len(nx) && supported_len(ny) && supported_len(nz), ERR_UNSUPPORTED,
                    "weighting needs template edges in the supported FFT lengths");
     if (!wsh_) {
-      TOMHIP_CHECK(hipMalloc(&wsh_, sizeof(float) * n3));
+      work_get(&wsh_, sizeof(float) * n3, s_);
       drop_graph();  // the captured batch reads wsh_
     }
     TOMHIP_CHECK(hipMemcpyAsync(wsh_, wsh, sizeof(float) * n3, hipMemcpyDefault, s_));
   } else if (wsh_) {
-    (void)hipFree(wsh_);
+    work_put(wsh_, s_);
     wsh_ = nullptr;
     drop_graph();
   }
@@ -1294,8 +1298,8 @@ void Search::run(const float* rm_host, long count, long first_index) {
   if (count <= 0) return;
   TOMHIP_REQUIRE(first_index >= 0 && first_index + count <= INT32_MAX, ERR_WRONG_INPUT, "angle index range");
   if (count > rm_cap_) {
-    (void)hipFree(rm_);
-    TOMHIP_CHECK(hipMalloc(&rm_, sizeof(float) * 9 * count));
+    work_put(rm_, s_);
+    work_get(&rm_, sizeof(float) * 9 * count, s_);
     rm_cap_ = count;
     drop_graph();  // captured pointers changed
   }
@@ -1317,7 +1321,7 @@ void Search::run(const float* rm_host, long count, long first_index) {
 
 void Search::capture_graph() {
   drop_graph();
-  if (!desc_) TOMHIP_CHECK(hipMalloc(&desc_, sizeof(long) * 2));
+  if (!desc_) work_get(&desc_, sizeof(long) * 2, s_);
   // twiddle tables are allocated on first use, which a capture does not allow
   for (int L : {nx, ny, nz, X, Y, Z, Xh}) (void)tw_.f32(L);
   if (use_fused(KA_)) fused_prepare(tw_, X, Y, Z);
@@ -1627,35 +1631,35 @@ void Search::refine(const float* volume, const float* rm_host, int G, int A, con
   float* cs = nullptr;
   int32_t *ca = nullptr, *cp = nullptr;
   auto release = [&] {
-    (void)hipFree(rm);
-    (void)hipFree(dshift);
-    (void)hipFree(cs);
-    (void)hipFree(ca);
-    (void)hipFree(cp);
+    work_put(rm, s_);
+    work_put(dshift, s_);
+    work_put(cs, s_);
+    work_put(ca, s_);
+    work_put(cp, s_);
   };
   try {
     if (centroid) {
-      TOMHIP_CHECK(hipMalloc(&dshift, sizeof(int32_t) * hshift.size()));
+      work_get(&dshift, sizeof(int32_t) * hshift.size(), s_);
       TOMHIP_CHECK(hipMemcpyAsync(dshift, hshift.data(), sizeof(int32_t) * hshift.size(), hipMemcpyHostToDevice, s_));
     }
-    TOMHIP_CHECK(hipMalloc(&rm, sizeof(float) * 9 * (long)G * A));
+    work_get(&rm, sizeof(float) * 9 * (long)G * A, s_);
     const long need = (long)KS * G * cb;  // templates per batch of chunks
     if (need > ref_cap_ || (wsh_ && !ref_work_)) {
       TOMHIP_CHECK(hipStreamSynchronize(s_));
-      (void)hipFree(ref_tt_);
-      (void)hipFree(ref_work_);
+      work_put(ref_tt_, s_);
+      work_put(ref_work_, s_);
       ref_tt_ = nullptr;
       ref_work_ = nullptr;
       ref_cap_ = 0;
-      TOMHIP_CHECK(hipMalloc(&ref_tt_, sizeof(float) * n3 * need));
-      if (wsh_) TOMHIP_CHECK(hipMalloc(&ref_work_, sizeof(c32) * n3 * need));
+      work_get(&ref_tt_, sizeof(float) * n3 * need, s_);
+      if (wsh_) work_get(&ref_work_, sizeof(c32) * n3 * need, s_);
       ref_cap_ = need;
     }
     float* tt = ref_tt_;
     c32* work = ref_work_;
-    TOMHIP_CHECK(hipMalloc(&cs, sizeof(float) * (long)nch * P));
-    TOMHIP_CHECK(hipMalloc(&ca, sizeof(int32_t) * (long)nch * P));
-    TOMHIP_CHECK(hipMalloc(&cp, sizeof(int32_t) * (long)nch * P));
+    work_get(&cs, sizeof(float) * (long)nch * P, s_);
+    work_get(&ca, sizeof(int32_t) * (long)nch * P, s_);
+    work_get(&cp, sizeof(int32_t) * (long)nch * P, s_);
     TOMHIP_CHECK(hipMemcpyAsync(rm, rm_host, sizeof(float) * 9 * (long)G * A, hipMemcpyHostToDevice, s_));
     // per-axis s - h of c[k] = sum_u t[u] V[k + u + s - h]
     const int sx = 2 * (X / 2) - X - nx / 2, sy = 2 * (Y / 2) - Y - ny / 2, sz = 2 * (Z / 2) - Z - nz / 2;

@@ -38,6 +38,7 @@
 #include "fft_kernels.h"
 #include "rotate.h"
 #include "rotate_dev.h"
+#include "pool.h"
 #include "subtomo.h"
 
 namespace tomhip {
@@ -696,7 +697,7 @@ void subtomo_run(Twiddles& tws, hipStream_t s, std::vector<SubtomoBox>& boxes_h,
   std::vector<void*> owned;
   auto alloc = [&](size_t bytes) {
     void* p = nullptr;
-    TOMHIP_CHECK(hipMalloc(&p, bytes));
+    work_get(&p, bytes, s);
     owned.push_back(p);
     return p;
   };
@@ -797,10 +798,10 @@ void subtomo_run(Twiddles& tws, hipStream_t s, std::vector<SubtomoBox>& boxes_h,
     }
     TOMHIP_CHECK(hipStreamSynchronize(s));
   } catch (...) {
-    for (void* p : owned) (void)hipFree(p);
+    for (void* p : owned) work_put(p, s);
     throw;
   }
-  for (void* p : owned) (void)hipFree(p);
+  for (void* p : owned) work_put(p, s);
 }
 
 }  // namespace tomhip

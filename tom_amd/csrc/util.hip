@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "fft_kernels.h"
+#include "pool.h"
 #include "util.h"
 
 namespace tomhip {
@@ -216,9 +217,9 @@ void prepare_template(Twiddles& tw, hipStream_t s, const float* T, int nx, int n
   double* t64 = nullptr;
   c64* c = nullptr;
   double* res = nullptr;
-  TOMHIP_CHECK(hipMalloc(&t64, sizeof(double) * n));
-  TOMHIP_CHECK(hipMalloc(&c, sizeof(c64) * n));
-  TOMHIP_CHECK(hipMalloc(&res, sizeof(double) * 2));
+  work_get(&t64, sizeof(double) * n, s);
+  work_get(&c, sizeof(c64) * n, s);
+  work_get(&res, sizeof(double) * 2, s);
   hipLaunchKernelGGL(k_tnorm, dim3(1), dim3(NTB), 0, s, T, n, t64, Tn32);
   hipLaunchKernelGGL(k_to_c64, dim3(gridn(n)), dim3(NT), 0, s, (const double*)t64, c, n);
   double scl = 1.0;
@@ -236,9 +237,9 @@ void prepare_template(Twiddles& tw, hipStream_t s, const float* T, int nx, int n
   TOMHIP_CHECK(hipStreamSynchronize(s));
   *mu_t = h[0];
   *sig_t = h[1];
-  (void)hipFree(t64);
-  (void)hipFree(c);
-  (void)hipFree(res);
+  work_put(t64, s);
+  work_put(c, s);
+  work_put(res, s);
 }
 
 void template_stats(hipStream_t s, const float* T, int nx, int ny, int nz, const float* M, double* mu_t,
@@ -246,8 +247,8 @@ void template_stats(hipStream_t s, const float* T, int nx, int ny, int nz, const
   const long n = (long)nx * ny * nz;
   c64* c = nullptr;
   double* res = nullptr;
-  TOMHIP_CHECK(hipMalloc(&c, sizeof(c64) * n));
-  TOMHIP_CHECK(hipMalloc(&res, sizeof(double) * 2));
+  work_get(&c, sizeof(c64) * n, s);
+  work_get(&res, sizeof(double) * 2, s);
   hipLaunchKernelGGL(k_f32_to_c64, dim3(gridn(n)), dim3(NT), 0, s, T, c, n);
   hipLaunchKernelGGL(k_norm_under_mask, dim3(1), dim3(NTB), 0, s, (const c64*)c, 1.0, M, n, res);
   TOMHIP_CHECK(hipGetLastError());
@@ -256,8 +257,8 @@ void template_stats(hipStream_t s, const float* T, int nx, int ny, int nz, const
   TOMHIP_CHECK(hipStreamSynchronize(s));
   *mu_t = h[0];
   *sig_t = h[1];
-  (void)hipFree(c);
-  (void)hipFree(res);
+  work_put(c, s);
+  work_put(res, s);
 }
 
 void launch_spheremask_os3(int nx, int ny, int nz, float* out, hipStream_t s) {
@@ -372,8 +373,8 @@ void global_max(const float* a, long n, float* val, long* idx, hipStream_t s) {
   const unsigned nb = gridn(n) > 1024 ? 1024 : gridn(n);
   float* pv = nullptr;
   long* pi = nullptr;
-  TOMHIP_CHECK(hipMalloc(&pv, sizeof(float) * nb));
-  TOMHIP_CHECK(hipMalloc(&pi, sizeof(long) * nb));
+  work_get(&pv, sizeof(float) * nb, s);
+  work_get(&pi, sizeof(long) * nb, s);
   hipLaunchKernelGGL(k_max_partial, dim3(nb), dim3(NT), 0, s, a, n, pv, pi);
   TOMHIP_CHECK(hipGetLastError());
   std::vector<float> hv(nb);
@@ -392,8 +393,8 @@ void global_max(const float* a, long n, float* val, long* idx, hipStream_t s) {
   }
   *val = bv;
   *idx = bi;
-  (void)hipFree(pv);
-  (void)hipFree(pi);
+  work_put(pv, s);
+  work_put(pi, s);
 }
 
 namespace {
