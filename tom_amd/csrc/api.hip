@@ -1105,8 +1105,7 @@ int tomhip_subtomo_score_batch(tomhip_ctx* ctx, int nbox, const int32_t* box_edg
       TOMHIP_REQUIRE(b.n > 0, ERR_WRONG_INPUT, "a mask has no non-zero voxel");
       b.M = dM.get<float>() + toff[k];
       b.Mcc = masks_cc ? dMcc.get<float>() + toff[k] : nullptr;
-      b.T = nullptr;
-      b.Tp = nullptr;
+      b.Tc = nullptr;
       b.FM = b.FB = nullptr;
     }
     // wedge tangents; rotation matrices
