@@ -26,7 +26,9 @@ void conv_fragments(const uint16_t* Wt, int Cout, int Cin, uint16_t* Wm, hipStre
 // dW[t][co][ci] += sum_v dY[v][co] X[v + d_t][ci]; dY bf16 [V][Cout].
 // (X chunk-planar when xq != 0, records of xs channels.)
 void conv_weight_grad(const uint16_t* X, int xs, int xo, long xq, int Cin, const uint16_t* dY, int Cout, int D, int H,
-                      int W, int taps, float* dW, hipStream_t s);
+                      int W, int taps, float* dW, float* part, hipStream_t s);
+// Elements of part, its scratch.
+long conv_weight_grad_elems(int Cin, int Cout, int D, int H, int W, int taps);
 
 class Unet {
  public:
