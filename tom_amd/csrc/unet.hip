@@ -657,35 +657,53 @@ __global__ void k_input(const float* vol, const float* aux, long V, uint16_t* X0
   }
 }
 
+// Gradient after an activation: channels [go, go + C) of rows of gs floats
+// and, where the activation was pooled, an eighth of the pooled voxel's row of
+// gp (the average pool's gradient; d: the activation's size).
+struct PostGrad {
+  const float* g;
+  int gs, go;
+  const float* gp;
+};
+
 // relu backward: dpre = dpost * (post > 0) -> bf16 for the MFMA, + bias
 // grad. Thread = 4 consecutive channels of a voxel (16-byte loads, 8-byte
 // stores); the thread count is a multiple of C / 4 so every thread keeps one
-// channel group and sums it, then the block adds its sums per channel.
-__global__ __launch_bounds__(NTU) void k_relu_bwd(const float* __restrict__ dpost, const uint16_t* __restrict__ post,
-                                                  int ps, int po, int C, long V, int relu, uint16_t* dpre,
-                                                  float* dbias) {
+// channel group and sums it, then the block adds its sums per channel. The
+// gradients of a skip connection and of the pool are added as they are read:
+// a pass each over the full-resolution gradient and its zeroing less (36, 27
+// and 6 us at 96^3).
+__global__ __launch_bounds__(NTU) void k_relu_bwd(PostGrad P, const uint16_t* __restrict__ post, int ps, int C,
+                                                  Dims d, uint16_t* dpre, float* dbias) {
   __shared__ float red[NTU][4];
   const int C4 = C / 4;
   const int per = NTU / C4;                 // voxels per block step
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, V = (int)d.V();
   float sum[4] = {0.f, 0.f, 0.f, 0.f};
   if (t < per * C4) {
     const int cg = t % C4;
-    for (long v = (long)blockIdx.x * per + t / C4; v < V; v += (long)gridDim.x * per) {
-      const float4 g = *reinterpret_cast<const float4*>(dpost + v * C + 4 * cg);
+    for (int v = blockIdx.x * per + t / C4; v < V; v += gridDim.x * per) {
+      const float4 g = *reinterpret_cast<const float4*>(P.g + (long)v * P.gs + P.go + 4 * cg);
+      const uint2 pr = *reinterpret_cast<const uint2*>(post + (long)v * ps + 4 * cg);
       float gv[4] = {g.x, g.y, g.z, g.w};
-      if (relu) {
-        const uint2 pr = *reinterpret_cast<const uint2*>(post + v * ps + po + 4 * cg);
-        const uint16_t pb[4] = {(uint16_t)(pr.x & 0xffffu), (uint16_t)(pr.x >> 16), (uint16_t)(pr.y & 0xffffu),
-                                (uint16_t)(pr.y >> 16)};
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if (!(bf2f(pb[k]) > 0.f)) gv[k] = 0.f;
+      if (P.gp) {
+        const int x = v % d.W, y = v / d.W % d.H, z = v / (d.W * d.H);
+        const long o = ((long)(z / 2) * (d.H / 2) + y / 2) * (d.W / 2) + x / 2;
+        const float4 q = *reinterpret_cast<const float4*>(P.gp + o * C + 4 * cg);
+        gv[0] += q.x * 0.125f;
+        gv[1] += q.y * 0.125f;
+        gv[2] += q.z * 0.125f;
+        gv[3] += q.w * 0.125f;
       }
+      const uint16_t pb[4] = {(uint16_t)(pr.x & 0xffffu), (uint16_t)(pr.x >> 16), (uint16_t)(pr.y & 0xffffu),
+                              (uint16_t)(pr.y >> 16)};
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (!(bf2f(pb[k]) > 0.f)) gv[k] = 0.f;
       uint2 o;
       o.x = (uint32_t)f2bf(gv[0]) | ((uint32_t)f2bf(gv[1]) << 16);
       o.y = (uint32_t)f2bf(gv[2]) | ((uint32_t)f2bf(gv[3]) << 16);
-      *reinterpret_cast<uint2*>(dpre + v * C + 4 * cg) = o;
+      *reinterpret_cast<uint2*>(dpre + (long)v * C + 4 * cg) = o;
 #pragma unroll
       for (int k = 0; k < 4; ++k) sum[k] += gv[k];
     }
@@ -731,22 +749,6 @@ __global__ __launch_bounds__(NTU) void k_pool(const uint16_t* __restrict__ X, in
   o.z = (uint32_t)f2bf(sum[4] * 0.125f) | ((uint32_t)f2bf(sum[5] * 0.125f) << 16);
   o.w = (uint32_t)f2bf(sum[6] * 0.125f) | ((uint32_t)f2bf(sum[7] * 0.125f) << 16);
   *reinterpret_cast<uint4*>(Y + (((long)z * oh + y) * ow + x) * C + c) = o;
-}
-
-// pool backward: dX (f32, [Vin][C], accumulated) += dY / 8 on each of the 8
-__global__ void k_pool_bwd(const float* dY, int C, Dims d, float* dX) {
-  const Dims o{d.D / 2, d.H / 2, d.W / 2};
-  const long n = o.V() * C;
-  for (long i = (long)blockIdx.x * NTU + threadIdx.x; i < n; i += (long)gridDim.x * NTU) {
-    const int c = (int)(i % C);
-    const long v = i / C;
-    const int x = (int)(v % o.W), y = (int)((v / o.W) % o.H), z = (int)(v / ((long)o.W * o.H));
-    const float g = dY[i] * 0.125f;
-    for (int k = 0; k < 8; ++k) {
-      const long s = (((long)(2 * z + (k >> 2)) * d.H + (2 * y + ((k >> 1) & 1))) * d.W + (2 * x + (k & 1)));
-      dX[s * C + c] += g;
-    }
-  }
 }
 
 // trilinear x2 upsampling (half-pixel centres, clamped), 1D weights per axis
@@ -866,108 +868,173 @@ __global__ __launch_bounds__(NTU) void k_up(const uint16_t* __restrict__ X, Dims
   }
 }
 
-// upsampling backward as a gather: dX[i] = sum over outputs using i
-__device__ __forceinline__ int up_back(int i, int n, int* o, float* w) {
-  int k = 0;
-  const int cand[4] = {2 * i - 1, 2 * i, 2 * i + 1, 2 * i + 2};
+// upsampling backward as a gather: dX[i] = sum over outputs using i, with
+// weight 0 (and an index inside) where fewer than four do
+__device__ __forceinline__ void up_back(int i, int n, int* o, float* w) {
+#pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int oo = cand[q];
-    if (oo < 0 || oo >= 2 * n) continue;
+    const int oo = 2 * i - 1 + q;
     int i0, i1;
     float w0, w1;
     up_taps(oo, n, &i0, &i1, &w0, &w1);
-    float ww = (i0 == i ? w0 : 0.f) + (i1 == i ? w1 : 0.f);
-    if (ww != 0.f) {
-      o[k] = oo;
-      w[k] = ww;
-      ++k;
+    const bool in = oo >= 0 && oo < 2 * n;
+    o[q] = in ? oo : 2 * i;
+    w[q] = in ? (i0 == i ? w0 : 0.f) + (i1 == i ? w1 : 0.f) : 0.f;
+  }
+}
+
+// dX[v][0 .. C) = the gather over channels [0, C) of dY's rows of ys floats.
+// Thread = 4 channels of a low-resolution voxel, so the 64 weights serve 4
+// sums and the loads are 16 bytes: 206 -> 90 us for 48^3 x 32 channels.
+__global__ __launch_bounds__(NTU) void k_up_bwd(const float* __restrict__ dY, int ys, int C, Dims lo, float* dX) {
+  const int HH = lo.H * 2, HW = lo.W * 2, C4 = C / 4;
+  const int i = blockIdx.x * NTU + threadIdx.x;
+  if (i >= (int)lo.V() * C4) return;
+  const int c = i % C4 * 4, v = i / C4;
+  const int x = v % lo.W, y = v / lo.W % lo.H, z = v / (lo.W * lo.H);
+  int xo[4], yo[4], zo[4];
+  float xw[4], yw[4], zw[4];
+  up_back(x, lo.W, xo, xw);
+  up_back(y, lo.H, yo, yw);
+  up_back(z, lo.D, zo, zw);
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const float* r = dY + ((long)zo[a] * HH + yo[b]) * HW * ys + c;
+      const float wzy = zw[a] * yw[b];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float4 g = *reinterpret_cast<const float4*>(r + (long)xo[e] * ys);
+        const float w = wzy * xw[e];
+        s.x += w * g.x;
+        s.y += w * g.y;
+        s.z += w * g.z;
+        s.w += w * g.w;
+      }
     }
-  }
-  return k;
-}
-
-__global__ void k_up_bwd(const float* dY, int ys, int yo, int C, Dims lo, float* dX) {
-  const Dims hi{lo.D * 2, lo.H * 2, lo.W * 2};
-  const long n = lo.V() * C;
-  for (long i = (long)blockIdx.x * NTU + threadIdx.x; i < n; i += (long)gridDim.x * NTU) {
-    const int c = (int)(i % C);
-    const long v = i / C;
-    const int x = (int)(v % lo.W), y = (int)((v / lo.W) % lo.H), z = (int)(v / ((long)lo.W * lo.H));
-    int xo[4], yo_[4], zo[4];
-    float xw[4], yw[4], zw[4];
-    const int nx = up_back(x, lo.W, xo, xw), ny = up_back(y, lo.H, yo_, yw), nz = up_back(z, lo.D, zo, zw);
-    float s = 0;
-    for (int a = 0; a < nz; ++a)
-      for (int b = 0; b < ny; ++b)
-        for (int e = 0; e < nx; ++e)
-          s += zw[a] * yw[b] * xw[e] * dY[(((long)zo[a] * hi.H + yo_[b]) * hi.W + xo[e]) * ys + yo + c];
-    dX[v * C + c] += s;
-  }
-}
-
-// split the gradient of a concatenated buffer: channels [off, off + C) of a
-// [V][Ctot] f32 gradient are added into dst [V][C]
-__global__ void k_split_add(const float* g, int Ctot, int off, int C, long V, float* dst) {
-  const long n = V * C;
-  for (long i = (long)blockIdx.x * NTU + threadIdx.x; i < n; i += (long)gridDim.x * NTU)
-    dst[i] += g[(i / C) * Ctot + off + (i % C)];
+  *reinterpret_cast<float4*>(dX + (long)v * C + c) = s;
 }
 
 // heads: logits [V][CH] f32; channel 0 particle logit, 1..nbin orientation.
 // Weighted BCE on channel 0 (mean over voxels), softmax CE over the bins at
-// voxels with a target bin (mean over those). Writes dlogits and loss sums.
-// Offsets: channels 1 + nbin .. 3 + nbin regress (centre - voxel) / 8 where
-// toff[v][3] > 0 (squared error, mean over those voxels).
-__global__ void k_loss(const float* logits, int CH, int nbin, const float* tprob, const int32_t* tbin,
-                       const float* toff, long V, float wpos, float inv_v, float inv_npos, float inv_noff,
-                       float* dlog, double* loss) {
+// voxels with a target bin (mean over those). Offsets: channels 1 + nbin ..
+// 3 + nbin regress (centre - voxel) / 8 where toff[v][3] > 0 (squared error,
+// mean over those voxels). Writes the logits' gradient in bf16 (the operand of
+// the head's gradients), adds its FP32 sums over the voxels to dbias and the
+// losses to loss.
+//
+// A wave takes 64 voxels: a lane each for channel 0, then all lanes together
+// for each voxel with a bin or offset target (a channel a lane: coalesced,
+// and the softmax sums are shuffles). The 64 rows are put together in LDS, where
+// they are zero but for the voxels that wrote to them, and stored in 16-byte
+// units. Bound by its writes, 160 bytes a voxel: 96^3 voxels 500 us (one
+// voxel a thread, FP32 rows) + 139 us (conversion and sums) -> 75 us.
+constexpr int LCH = 80;
+__global__ __launch_bounds__(NTU) void k_loss(const float* __restrict__ logits, int nbin,
+                                              const float* __restrict__ tprob, const int32_t* __restrict__ tbin,
+                                              const float* __restrict__ toff, long V, float wpos, float inv_v,
+                                              float inv_npos, float inv_noff, uint16_t* __restrict__ dlog,
+                                              float* dbias, double* loss) {
+  __shared__ uint4 tile4[NTU / 64][64 * LCH / 8];
+  __shared__ float bsum[NTU / 64][LCH];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  uint16_t* tile = reinterpret_cast<uint16_t*>(tile4[wv]);
+  for (int i = lane; i < 64 * LCH / 8; i += 64) tile4[wv][i] = make_uint4(0, 0, 0, 0);
   double l1 = 0, l2 = 0, l3 = 0;
+  float b0 = 0.f, bc[2] = {0.f, 0.f};  // sums of channel 0; of channels 1 + lane, 65 + lane
   const int oc = 1 + nbin;
-  for (long v = (long)blockIdx.x * NTU + threadIdx.x; v < V; v += (long)gridDim.x * NTU) {
-    const float* L = logits + v * CH;
-    float* G = dlog + v * CH;
-    const float z = L[0], t = tprob[v];
+  for (long v0 = ((long)blockIdx.x * (NTU / 64) + wv) * 64; v0 < V; v0 += (long)gridDim.x * NTU) {
+    const int rows = (int)min(64L, V - v0);
+    const bool in = lane < rows;
+    const long v = in ? v0 + lane : v0;
+    const float z = logits[v * LCH], t = tprob[v];
+    const int b = in && tbin ? tbin[v] : -1;
+    float4 off = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (toff && in) off = make_float4(toff[v * 4], toff[v * 4 + 1], toff[v * 4 + 2], toff[v * 4 + 3]);
     const float p = 1.f / (1.f + expf(-z));
     // -[wpos t log p + (1-t) log(1-p)], stable
     const float lp = -log1pf(expf(-fabsf(z))) + fminf(z, 0.f);   // log p
     const float lq = -log1pf(expf(-fabsf(z))) + fminf(-z, 0.f);  // log(1-p)
-    l1 += -(wpos * t * lp + (1.f - t) * lq);
-    G[0] = (wpos * t * (p - 1.f) + (1.f - t) * p) * inv_v;
-    for (int c = 1; c < CH; ++c) G[c] = 0.f;
-    const int b = tbin ? tbin[v] : -1;
-    if (b >= 0 && b < nbin) {
-      float mx = -FLT_MAX;
-      for (int c = 0; c < nbin; ++c) mx = fmaxf(mx, L[1 + c]);
-      float se = 0;
-      for (int c = 0; c < nbin; ++c) se += expf(L[1 + c] - mx);
-      l2 += -(L[1 + b] - mx - logf(se));
-      for (int c = 0; c < nbin; ++c) G[1 + c] = (expf(L[1 + c] - mx) / se - (c == b ? 1.f : 0.f)) * inv_npos;
-    }
-    if (toff && toff[v * 4 + 3] > 0.f) {
-      for (int c = 0; c < 3; ++c) {
-        const float d = L[oc + c] - toff[v * 4 + c];
-        l3 += (double)d * d;
-        G[oc + c] = 2.f * d * inv_noff;
+    const float g0 = in ? (wpos * t * (p - 1.f) + (1.f - t) * p) * inv_v : 0.f;
+    if (in) l1 += -(wpos * t * lp + (1.f - t) * lq);
+    b0 += g0;
+    tile[lane * LCH] = f2bf(g0);
+    const bool hasb = b >= 0 && b < nbin, haso = off.w > 0.f;
+    const unsigned long long todo = __ballot(hasb || haso);
+    for (unsigned long long m = todo; m; m &= m - 1) {
+      const int r = __builtin_ctzll(m);
+      const float* L = logits + (v0 + r) * LCH;
+      const int br = __shfl(b, r, 64);
+      float g[2] = {0.f, 0.f};
+      if (br >= 0 && br < nbin) {
+        const float x0 = lane < nbin ? L[1 + lane] : -FLT_MAX;
+        const float x1 = lane + 64 < nbin ? L[65 + lane] : -FLT_MAX;
+        float mx = fmaxf(x0, x1);
+        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+        const float e0 = lane < nbin ? expf(x0 - mx) : 0.f, e1 = lane + 64 < nbin ? expf(x1 - mx) : 0.f;
+        float se = e0 + e1;
+        for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
+        if (br < 64 ? lane == br : lane + 64 == br) l2 += -((br < 64 ? x0 : x1) - mx - logf(se));
+        if (lane < nbin) g[0] = (e0 / se - (lane == br ? 1.f : 0.f)) * inv_npos;
+        if (lane + 64 < nbin) g[1] = (e1 / se - (lane + 64 == br ? 1.f : 0.f)) * inv_npos;
       }
+      const float ox = __shfl(off.x, r, 64), oy = __shfl(off.y, r, 64), oz = __shfl(off.z, r, 64);
+      if (__shfl(off.w, r, 64) > 0.f) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int c = 1 + 64 * h + lane - oc;  // offset channel of this lane
+          if (c >= 0 && c < 3) {
+            const float d = L[oc + c] - (c == 0 ? ox : c == 1 ? oy : oz);
+            l3 += (double)d * d;
+            g[h] = 2.f * d * inv_noff;
+          }
+        }
+      }
+      tile[r * LCH + 1 + lane] = f2bf(g[0]);
+      if (lane < LCH - 65) tile[r * LCH + 65 + lane] = f2bf(g[1]);
+      bc[0] += g[0];
+      bc[1] += g[1];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint4* out = reinterpret_cast<uint4*>(dlog + v0 * LCH);
+    for (int i = lane; i < rows * (LCH / 8); i += 64) out[i] = tile4[wv][i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (unsigned long long m = todo; m; m &= m - 1) {
+      const int r = __builtin_ctzll(m);
+      tile[r * LCH + 1 + lane] = 0;
+      if (lane < LCH - 65) tile[r * LCH + 65 + lane] = 0;
     }
   }
   for (int o = 32; o > 0; o >>= 1) {
     l1 += __shfl_xor(l1, o, 64);
     l2 += __shfl_xor(l2, o, 64);
     l3 += __shfl_xor(l3, o, 64);
+    b0 += __shfl_xor(b0, o, 64);
   }
-  // one set of FP64 atomics per block (the grid is capped at a few hundred)
+  // one set of atomics per block (the grid is capped at a thousand)
   __shared__ double red[3][NTU / 64];
-  if ((threadIdx.x & 63) == 0) {
-    red[0][threadIdx.x >> 6] = l1;
-    red[1][threadIdx.x >> 6] = l2;
-    red[2][threadIdx.x >> 6] = l3;
+  if (lane == 0) {
+    red[0][wv] = l1;
+    red[1][wv] = l2;
+    red[2][wv] = l3;
+    bsum[wv][0] = b0;
   }
+  bsum[wv][1 + lane] = bc[0];
+  if (lane < LCH - 65) bsum[wv][65 + lane] = bc[1];
   __syncthreads();
   if (threadIdx.x < 3) {
     double a = 0;
     for (int w = 0; w < NTU / 64; ++w) a += red[threadIdx.x][w];
     atomicAdd(&loss[threadIdx.x], a);
+  }
+  if (threadIdx.x < LCH) {
+    float a = 0;
+    for (int w = 0; w < NTU / 64; ++w) a += bsum[w][threadIdx.x];
+    atomicAdd(&dbias[threadIdx.x], a);
   }
 }
 
@@ -1399,8 +1466,7 @@ struct Unet::Impl {
   uint16_t *x0, *a1, *c1, *p1, *a2, *c2, *p2, *b1, *b2, *d2a, *d2b, *d1a, *d1b;
   float* logits;
   // gradients (f32) and bf16 pre-activation gradients
-  float *g_logits, *g_d1b, *g_d1a, *g_c1, *g_d2b, *g_d2a, *g_c2, *g_b2, *g_b1, *g_p2, *g_s2, *g_a2, *g_p1, *g_s1,
-      *g_a1;
+  float *g_d1b, *g_d1a, *g_c1, *g_d2b, *g_d2a, *g_c2, *g_b2, *g_b1, *g_p2, *g_a2, *g_p1, *g_a1;
   float* dwp;    // scratch: parts of a weight gradient
   uint16_t* gb;  // scratch bf16 pre-activation gradient (largest: V0 * 80)
   double* loss;
@@ -1502,7 +1568,6 @@ Unet::Unet(hipStream_t s, int D, int H, int W, int nbin, uint64_t seed, bool tra
     TOMHIP_CHECK(hipStreamSynchronize(s));
     return;
   }
-  I.g_logits = I.alloc<float>(V0 * kHeadCh);
   I.g_d1b = I.alloc<float>(V0 * 16);
   I.g_d1a = I.alloc<float>(V0 * 16);
   I.g_c1 = I.alloc<float>(V0 * 48);
@@ -1512,10 +1577,8 @@ Unet::Unet(hipStream_t s, int D, int H, int W, int nbin, uint64_t seed, bool tra
   I.g_b2 = I.alloc<float>(V2 * 64);
   I.g_b1 = I.alloc<float>(V2 * 64);
   I.g_p2 = I.alloc<float>(V2 * 32);
-  I.g_s2 = I.alloc<float>(V1 * 32);
   I.g_a2 = I.alloc<float>(V1 * 32);
   I.g_p1 = I.alloc<float>(V1 * 16);
-  I.g_s1 = I.alloc<float>(V0 * 16);
   I.g_a1 = I.alloc<float>(V0 * 16);
   I.gb = I.alloc<uint16_t>(V0 * kHeadCh);
   long dwp = 0;
@@ -1705,57 +1768,49 @@ void Unet::backward(const float* tprob, const int32_t* tbin, const float* toff, 
   for (auto& c : L) TOMHIP_CHECK(hipMemsetAsync(c.g, 0, sizeof(float) * c.np, s));
   const float inv_v = 1.f / (float)I.V0, inv_np = npos > 0 ? 1.f / (float)npos : 0.f;
   const float inv_no = noff > 0 ? 1.f / (float)noff : 0.f;
-  hipLaunchKernelGGL(k_loss, dim3(std::min(gridv(I.V0), 512u)), dim3(NTU), 0, s, (const float*)I.logits, kHeadCh, I.nbin, tprob,
-                     tbin, toff, I.V0, wpos, inv_v, inv_np, inv_no, I.g_logits, I.loss);
-  // zero the accumulated data gradients
-  auto zero = [&](float* p, long n) { TOMHIP_CHECK(hipMemsetAsync(p, 0, sizeof(float) * n, s)); };
-  zero(I.g_c1, I.V0 * 48);
-  zero(I.g_c2, I.V1 * 96);
-  zero(I.g_s1, I.V0 * 16);
-  zero(I.g_s2, I.V1 * 32);
-  zero(I.g_b2, I.V2 * 64);
-  zero(I.g_d2b, I.V1 * 32);
-  // one layer: gpost (f32 [V][Cout]) + its post-activation -> weight/bias
-  // grads and (optionally) the data gradient into gin (f32, [V][Cin]) at
-  // channel stride gs
+  static_assert(kHeadCh == LCH, "k_loss's rows");
+  hipLaunchKernelGGL(k_loss, dim3(std::min(gridv(I.V0), 1024u)), dim3(NTU), 0, s, (const float*)I.logits, I.nbin, tprob,
+                     tbin, toff, I.V0, wpos, inv_v, inv_np, inv_no, I.gb, L[10].g + 16L * kHeadCh, I.loss);
+  // a layer's pre-activation gradient in gb -> weight gradient and
+  // (optionally) the data gradient into gin (f32 [V][Cin])
   const long q1 = I.V0 * 16, q2 = I.V1 * 32;
   const uint16_t* skip1 = I.c1 + 2 * q1;
   const uint16_t* skip2 = I.c2 + 2 * q2;
-  auto layer_bwd = [&](int li, const float* gpost, const uint16_t* post, int ps, int po, const uint16_t* X, int xs,
-                       int xo, long xq, Dims d, float* gin) {
+  auto products = [&](int li, const uint16_t* X, int xs, long xq, Dims d, float* gin) {
     ConvLayer& c = L[li];
-    const long V = d.V();
-    const dim3 g(gridv(V) > 2048 ? 2048 : gridv(V));
-    hipLaunchKernelGGL(k_relu_bwd, g, dim3(NTU), 0, s, gpost, post, ps, po, c.Cout, V, c.relu, I.gb,
-                       c.g + (long)c.taps * c.Cout * c.Cin);
-    conv_weight_grad(X, xs, xo, xq, c.Cin, I.gb, c.Cout, d.D, d.H, d.W, c.taps, c.g, I.dwp, s);
+    conv_weight_grad(X, xs, 0, xq, c.Cin, I.gb, c.Cout, d.D, d.H, d.W, c.taps, c.g, I.dwp, s);
     if (gin)
       conv_forward(I.gb, c.Cout, 0, 0, c.Cout, d.D, d.H, d.W, c.wf, c.wfm, nullptr, c.Cin, c.taps, 0, nullptr, 0, 0,
                    gin, s);
   };
-  // head (no relu; post unused)
-  layer_bwd(10, I.g_logits, I.d1b, 16, 0, I.d1b, 16, 0, 0, d0, I.g_d1b);
-  layer_bwd(9, I.g_d1b, I.d1b, 16, 0, I.d1a, 16, 0, 0, d0, I.g_d1a);
-  layer_bwd(8, I.g_d1a, I.d1a, 16, 0, I.c1, 16, 0, q1, d0, I.g_c1);
-  // c1 = [up(d2b) | skip1]
-  hipLaunchKernelGGL(k_split_add, dim3(gridv(I.V0 * 16)), dim3(NTU), 0, s, (const float*)I.g_c1, 48, 32, 16, I.V0,
-                     I.g_s1);
-  hipLaunchKernelGGL(k_up_bwd, dim3(gridv(I.V1 * 32)), dim3(NTU), 0, s, (const float*)I.g_c1, 48, 0, 32, d1,
-                     I.g_d2b);
-  layer_bwd(7, I.g_d2b, I.d2b, 32, 0, I.d2a, 32, 0, 0, d1, I.g_d2a);
-  layer_bwd(6, I.g_d2a, I.d2a, 32, 0, I.c2, 32, 0, q2, d1, I.g_c2);
-  hipLaunchKernelGGL(k_split_add, dim3(gridv(I.V1 * 32)), dim3(NTU), 0, s, (const float*)I.g_c2, 96, 64, 32, I.V1,
-                     I.g_s2);
-  hipLaunchKernelGGL(k_up_bwd, dim3(gridv(I.V2 * 64)), dim3(NTU), 0, s, (const float*)I.g_c2, 96, 0, 64, d2,
-                     I.g_b2);
-  layer_bwd(5, I.g_b2, I.b2, 64, 0, I.b1, 64, 0, 0, d2, I.g_b1);
-  layer_bwd(4, I.g_b1, I.b1, 64, 0, I.p2, 32, 0, 0, d2, I.g_p2);
-  hipLaunchKernelGGL(k_pool_bwd, dim3(gridv(I.V2 * 32)), dim3(NTU), 0, s, (const float*)I.g_p2, 32, d1, I.g_s2);
-  layer_bwd(3, I.g_s2, skip2, 32, 0, I.a2, 32, 0, 0, d1, I.g_a2);
-  layer_bwd(2, I.g_a2, I.a2, 32, 0, I.p1, 16, 0, 0, d1, I.g_p1);
-  hipLaunchKernelGGL(k_pool_bwd, dim3(gridv(I.V1 * 16)), dim3(NTU), 0, s, (const float*)I.g_p1, 16, d0, I.g_s1);
-  layer_bwd(1, I.g_s1, skip1, 16, 0, I.a1, 16, 0, 0, d0, I.g_a1);
-  layer_bwd(0, I.g_a1, I.a1, 16, 0, I.x0, 16, 0, 0, d0, nullptr);
+  // one layer: the gradient after its activation -> pre-activation and bias
+  auto layer_bwd = [&](int li, PostGrad gpost, const uint16_t* post, const uint16_t* X, int xs, long xq, Dims d,
+                       float* gin) {
+    ConvLayer& c = L[li];
+    const unsigned g = gridv(d.V());
+    hipLaunchKernelGGL(k_relu_bwd, dim3(g > 2048 ? 2048 : g), dim3(NTU), 0, s, gpost, post, c.Cout, c.Cout, d, I.gb,
+                       c.g + (long)c.taps * c.Cout * c.Cin);
+    products(li, X, xs, xq, d, gin);
+  };
+  auto plain = [&](const float* g, int C) { return PostGrad{g, C, 0, nullptr}; };
+  // gradient of the up-sampled channels [0, C) of a concatenation
+  auto up_bwd = [&](const float* g, int ys, int C, Dims lo, float* out) {
+    hipLaunchKernelGGL(k_up_bwd, dim3((unsigned)((lo.V() * (C / 4) + NTU - 1) / NTU)), dim3(NTU), 0, s, g, ys, C, lo,
+                       out);
+  };
+  products(10, I.d1b, 16, 0, d0, I.g_d1b);  // head (no relu)
+  layer_bwd(9, plain(I.g_d1b, 16), I.d1b, I.d1a, 16, 0, d0, I.g_d1a);
+  layer_bwd(8, plain(I.g_d1a, 16), I.d1a, I.c1, 16, q1, d0, I.g_c1);
+  up_bwd(I.g_c1, 48, 32, d1, I.g_d2b);  // c1 = [up(d2b) | skip1]
+  layer_bwd(7, plain(I.g_d2b, 32), I.d2b, I.d2a, 32, 0, d1, I.g_d2a);
+  layer_bwd(6, plain(I.g_d2a, 32), I.d2a, I.c2, 32, q2, d1, I.g_c2);
+  up_bwd(I.g_c2, 96, 64, d2, I.g_b2);  // c2 = [up(b2) | skip2]
+  layer_bwd(5, plain(I.g_b2, 64), I.b2, I.b1, 64, 0, d2, I.g_b1);
+  layer_bwd(4, plain(I.g_b1, 64), I.b1, I.p2, 32, 0, d2, I.g_p2);
+  layer_bwd(3, PostGrad{I.g_c2, 96, 64, I.g_p2}, skip2, I.a2, 32, 0, d1, I.g_a2);
+  layer_bwd(2, plain(I.g_a2, 32), I.a2, I.p1, 16, 0, d1, I.g_p1);
+  layer_bwd(1, PostGrad{I.g_c1, 48, 32, I.g_p1}, skip1, I.a1, 16, 0, d0, I.g_a1);
+  layer_bwd(0, plain(I.g_a1, 16), I.a1, I.x0, 16, 0, d0, nullptr);
   TOMHIP_CHECK(hipGetLastError());
   if (loss_out) {
     double h[3];
