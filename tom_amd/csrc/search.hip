@@ -345,7 +345,7 @@ __global__ __launch_bounds__(NTT) void k_tmpl_fwd_y(const c32* Tx, c32* Ty, c32*
 }
 
 // ---------------------------------------------------------------- pass A
-// grid (Xh/TW, Y), 512 threads. For each angle of the batch: z forward FFT of
+// 512 threads. For each of its angles: z forward FFT of
 // the template lines (stage 0 reads the n non-zero planes straight from Ty),
 // product with F_I in the last forward stage, Nyquist packing, z inverse FFT
 // whose last stage writes Q directly. F_I stays in LDS across the batch when
@@ -356,9 +356,10 @@ constexpr bool passA_fi_lds() {
   return (2 * Z * (TW + 1) + Z) * 8 <= 150 * 1024;
 }
 
+// grid (Xh / TW - 1 or 1, Y, groups of apb angles)
 template <int Z, int TW, bool NYQ>
 __global__ __launch_bounds__(NT_A) void k_passA(const c32* Ty, const c32* Tyn, const c32* FI, const c32* FIn,
-                                                c32* Q, const c32* twZg, int Y, int Xh, int nz, int ka) {
+                                                c32* Q, const c32* twZg, int Y, int Xh, int nz, int ka, int apb) {
   // NYQ: the kx tile 0 launch, which also carries the kx = X/2 line (line TW)
   constexpr int P = TW + 1;
   constexpr int NL = NYQ ? P : TW;
@@ -370,6 +371,7 @@ __global__ __launch_bounds__(NT_A) void k_passA(const c32* Ty, const c32* Tyn, c
   __shared__ c32 fis[FL ? E : 1];
   __shared__ c32 twZ[Z];
   const int tile = NYQ ? 0 : blockIdx.x + 1, ky = blockIdx.y;
+  const int a0 = blockIdx.z * apb, a1 = min(a0 + apb, ka);
   load_table<float, Z, NT_A>(twZ, twZg);
   auto fi_at = [&](int c, int kz) -> c32 {
     if (!NYQ || c < TW) return FI[((long)kz * Y + ky) * Xh + tile * TW + c];
@@ -412,8 +414,8 @@ __global__ __launch_bounds__(NT_A) void k_passA(const c32* Ty, const c32* Tyn, c
       }
     }
   };
-  fetch(0);
-  for (int a = 0; a < ka; ++a) {
+  fetch(a0);
+  for (int a = a0; a < a1; ++a) {
     auto prod = [&](int c, int kz, c32 v) -> c32 {
       if constexpr (FL)
         return cmulc(fis[kz * P + c], v);
@@ -434,7 +436,7 @@ __global__ __launch_bounds__(NT_A) void k_passA(const c32* Ty, const c32* Tyn, c
           for (int r = 0; r < I0::R; ++r) buf[Lay::addr(line, j * I0::R + r)] = v[r];
         }
       }
-      if (a + 1 < ka) fetch(a + 1);
+      if (a + 1 < a1) fetch(a + 1);
       __syncthreads();
     } else {
       stage0_g2l<float, Z, NL, NT_A, -1, Lay>(buf, [&](int c, int z) { return ld_at(a, c, z); });
@@ -580,18 +582,21 @@ constexpr int passc_lines() {
 }
 constexpr int NT_C = 512;
 
-// grid (ceil(Y*Z / NL)). Half-length c2r along x of every angle of the batch.
+// grid (ceil(Y*Z / NL), groups of apb angles). Half-length c2r along x of the
+// group's angles.
 // Stage 0 reads each butterfly j together with its mirror NJ0 - j, so the
 // real-to-complex pre-twiddle Z'[k] = A + iB, Z'[XH-k] = conj(A) + i conj(B),
 //   A = G[k] + conj(G[XH-k]),  B = (G[k] - conj(G[XH-k])) e^{2πik/X},
 // (G[0], G[X/2] packed in column 0) happens in registers. The last stage feeds
 // a per-thread running max/argmax over the batch; one compare/update of the
 // resident maps follows.
-template <int XH>
+template <int XH, bool GROUPS>
 __global__ __launch_bounds__(NT_C) __attribute__((amdgpu_waves_per_eu(4))) void k_passC(const c32* Q, float* maxc, int32_t* argm, const c32* twHg,
                                                 const c32* twXg, long line0, long nlines, long qstride, int ka,
-                                                int first_index, const long* desc) {
+                                                int first_index, const long* desc, int apb, float* pv, uint8_t* pi,
+                                                long n) {
   if (desc) first_index = (int)(desc[1] + desc[0] * ka);
+  const int a0 = GROUPS ? blockIdx.y * apb : 0, a1 = GROUPS ? min(a0 + apb, ka) : ka;
   constexpr int NL = passc_lines<XH>();
   constexpr int S = plan_nstages(XH);
   constexpr int R0 = plan_radix(XH, 0);
@@ -640,14 +645,25 @@ __global__ __launch_bounds__(NT_C) __attribute__((amdgpu_waves_per_eu(4))) void 
       pf[k] = (i < nvv) ? src4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
   };
-  fetch(0);
-  for (int a = 0; a < ka; ++a) {
+  // The batch's first angle is taken whatever it is; the other groups start
+  // below every value, so that merging them in order takes what a run through
+  // the batch takes.
+  if constexpr (GROUPS) {
+#pragma unroll
+    for (int p = 0; p < IN::PER; ++p) {
+      ix[p] = iy[p] = 0u;
+#pragma unroll
+      for (int r = 0; r < IN::R; ++r) bx[p][r] = by[p][r] = -INFINITY;
+    }
+  }
+  fetch(a0);
+  for (int a = a0; a < a1; ++a) {
 #pragma unroll
     for (int k = 0; k < PF; ++k) {
       const int i = threadIdx.x + k * NT_C;  // float4 i: row i / (XH/2), elements 2 (i % (XH/2)) + 0, 1
       if (i < NV) reinterpret_cast<float4*>(raw + (i / (XH / 2)) * RP)[i % (XH / 2)] = pf[k];
     }
-    if (a + 1 < ka) fetch(a + 1);
+    if (a + 1 < a1) fetch(a + 1);
     __syncthreads();
 #pragma unroll 1
     for (int p = 0; p < PERT; ++p) {
@@ -710,7 +726,7 @@ __global__ __launch_bounds__(NT_C) __attribute__((amdgpu_waves_per_eu(4))) void 
     }
     __syncthreads();
     StagesL2L<float, XH, 1, S - 1, NL, NT_C, 1, Lay>::run(buf, twH);
-    if (a == 0) {
+    if (!GROUPS && a == 0) {
 #pragma unroll
       for (int p = 0; p < IN::PER; ++p) ix[p] = iy[p] = 0u;
     }
@@ -740,8 +756,8 @@ __global__ __launch_bounds__(NT_C) __attribute__((amdgpu_waves_per_eu(4))) void 
       for (int r = 0; r < IN::R; ++r) {
         const int e = line * FP + j + r * IN::NS;
         sval[e] = make_float2(bx[p][r], by[p][r]);
-        sidx[e] = make_int2(first_index + (int)((ix[p] >> (4 * r)) & 15u),
-                            first_index + (int)((iy[p] >> (4 * r)) & 15u));
+        const int first = GROUPS ? 0 : first_index;
+        sidx[e] = make_int2(first + (int)((ix[p] >> (4 * r)) & 15u), first + (int)((iy[p] >> (4 * r)) & 15u));
       }
     }
   }
@@ -749,9 +765,14 @@ __global__ __launch_bounds__(NT_C) __attribute__((amdgpu_waves_per_eu(4))) void 
   for (int i = threadIdx.x; i < nlv * XH; i += NT_C) {
     const int line = i / XH, e = i % XH;
     const long v = ((l0 + line) * XH + e) * 2;
-    const float2 cur = *reinterpret_cast<const float2*>(maxc + v);
     const float2 nv = sval[line * FP + e];
     const int2 ni = sidx[line * FP + e];
+    if constexpr (GROUPS) {  // merged by k_merge_groups
+      *reinterpret_cast<float2*>(pv + blockIdx.y * n + v) = nv;
+      *reinterpret_cast<uchar2*>(pi + blockIdx.y * n + v) = make_uchar2(ni.x, ni.y);
+      continue;
+    }
+    const float2 cur = *reinterpret_cast<const float2*>(maxc + v);
     if (nv.x > cur.x) {
       maxc[v] = nv.x;
       argm[v] = ni.x;
@@ -760,6 +781,40 @@ __global__ __launch_bounds__(NT_C) __attribute__((amdgpu_waves_per_eu(4))) void 
       maxc[v + 1] = nv.y;
       argm[v + 1] = ni.y;
     }
+  }
+}
+
+// The groups' maxima in order against the resident maps, voxels v0 .. v0 + cnt
+// - 1 (both even), two a thread.
+__global__ __launch_bounds__(NT) void k_merge_groups(const float* __restrict__ pv, const uint8_t* __restrict__ pi,
+                                                     int groups, long n, long v0, long cnt, int first_index,
+                                                     const long* desc, int ka, float* maxc, int32_t* argm) {
+  if (desc) first_index = (int)(desc[1] + desc[0] * ka);
+  const long i = ((long)blockIdx.x * NT + threadIdx.x) * 2;
+  if (i >= cnt) return;
+  const long v = v0 + i;
+  float2 b = *reinterpret_cast<const float2*>(pv + v);
+  uchar2 x = *reinterpret_cast<const uchar2*>(pi + v);
+  for (int g = 1; g < groups; ++g) {
+    const float2 c = *reinterpret_cast<const float2*>(pv + g * n + v);
+    const uchar2 y = *reinterpret_cast<const uchar2*>(pi + g * n + v);
+    if (c.x > b.x) {
+      b.x = c.x;
+      x.x = y.x;
+    }
+    if (c.y > b.y) {
+      b.y = c.y;
+      x.y = y.y;
+    }
+  }
+  const float2 cur = *reinterpret_cast<const float2*>(maxc + v);
+  if (b.x > cur.x) {
+    maxc[v] = b.x;
+    argm[v] = first_index + x.x;
+  }
+  if (b.y > cur.y) {
+    maxc[v + 1] = b.y;
+    argm[v + 1] = first_index + x.y;
   }
 }
 
@@ -1047,6 +1102,10 @@ Search::Search(Twiddles& tw, hipStream_t s, const float* volume, int X_, int Y_,
     work_get(&Tyn_, sizeof(c32) * (long)KA_ * nz * Y, s_);
     work_get(&Q_, sizeof(c32) * (long)KA_ * Z * Y * Xh, s_);
     if (fused_supported(X, Y, Z, KA_)) work_get(&Pn_, sizeof(c32) * (long)KA_ * Z * Y, s_);
+    if (const long g = passC_groups(KA_); g > 1) {
+      work_get(&gmax_, sizeof(float) * g * N, s_);
+      work_get(&garg_, g * N, s_);
+    }
     // the template's x-DFT rows live in Q between the template forward and
     // pass A, unless the template is as large as the volume in y and z
     const long txn = (long)KA_ * nz * ny * tx_pitch(Xh);
@@ -1099,6 +1158,8 @@ void Search::release() {
   work_put_idle(Tx_);
   work_put_idle(Q_);
   work_put_idle(Pn_);
+  work_put_idle(gmax_);
+  work_put_idle(garg_);
   work_put_idle(mu_);
   work_put_idle(sig_);
   work_put_idle(wsh_);
@@ -1111,6 +1172,8 @@ void Search::release() {
   argm_ = nullptr;
   tmpl_ = t1_ = wsh_ = rm_ = ref_tt_ = nullptr;
   tbox_ = Ty_ = Tyn_ = Tx_ = Q_ = Pn_ = ref_work_ = nullptr;
+  gmax_ = nullptr;
+  garg_ = nullptr;
   mu_ = sig_ = nullptr;
   mask_ = nullptr;
   drop_graph();
@@ -1463,11 +1526,20 @@ void Search::launch_passA(int ka) {
           hipLaunchKernelGGL(k_passA4<false>, dim3(Xh / TW - 1, Y), dim3(256), 0, s_, (const c32*)Ty_,
                              (const c32*)Tyn_, (const c32*)FI_, (const c32*)FIn_, Q_, tw_.f32(L), Y, Xh, nz, ka);
       } else if constexpr ((long)L * (TW + 1) * 8 + (long)L * 8 <= kLdsMax) {
-        hipLaunchKernelGGL((k_passA<L, TW, true>), dim3(1, Y), dim3(NT_A), 0, s_, (const c32*)Ty_, (const c32*)Tyn_,
-                           (const c32*)FI_, (const c32*)FIn_, Q_, tw_.f32(L), Y, Xh, nz, ka);
-        if (Xh > TW)
-          hipLaunchKernelGGL((k_passA<L, TW, false>), dim3(Xh / TW - 1, Y), dim3(NT_A), 0, s_, (const c32*)Ty_,
-                             (const c32*)Tyn_, (const c32*)FI_, (const c32*)FIn_, Q_, tw_.f32(L), Y, Xh, nz, ka);
+        // few blocks: spread the batch's angles over as many as the CUs hold
+        // at once. Batches of 16, undivided and divided, in us: 64x64x64 68
+        // and 29, 128x128x64 68 and 50. One launch for both kinds of tile
+        // takes 20 at 64x64x64 but 67 for 61 at 320x240x96 ka 4.
+        constexpr long lds = (passA_fi_lds<L, TW>() ? 2 : 1) * (long)L * (TW + 1) * 8 + L * 8;
+        constexpr int per_cu = (int)std::min(2048L / NT_A, 160 * 1024 / lds);
+        auto go = [&](auto kern, int tiles) {
+          const int groups = std::min(ka, std::max(1, 256 * per_cu / (tiles * Y)));
+          const int apb = (ka + groups - 1) / groups;
+          hipLaunchKernelGGL(kern, dim3(tiles, Y, (ka + apb - 1) / apb), dim3(NT_A), 0, s_, (const c32*)Ty_,
+                             (const c32*)Tyn_, (const c32*)FI_, (const c32*)FIn_, Q_, tw_.f32(L), Y, Xh, nz, ka, apb);
+        };
+        go(k_passA<L, TW, true>, 1);
+        if (Xh > TW) go(k_passA<L, TW, false>, Xh / TW - 1);
       } else {
         throw Error(ERR_UNSUPPORTED, "pass A tile does not fit in LDS");
       }
@@ -1559,14 +1631,43 @@ void Search::run_batch(const float* rm_dev, int ka, long first_index, const long
   }
 }
 
+// Angle groups of pass C: with few blocks a batch's angles, one after the
+// other in each of them, take longer than their data. As many groups as give
+// each CU a block, two angles or more each, merged by one more launch.
+// Batches of 16, undivided and divided with the merge, in us: 64x64x64 (32
+// blocks) 34 and 17, 128x128x64 (128 blocks) 38 and 25.
+int Search::passC_groups(int ka) const {
+  int groups = 1;
+  dispatch_xh(Xh, [&](auto Lc) {
+    constexpr int NL = passc_lines<decltype(Lc)::value>();
+    const long blocks = ((long)Z * Y + NL - 1) / NL;
+    groups = (int)std::max(1L, std::min((long)ka / 2, 256 / blocks));
+  });
+  return groups;
+}
+
 void Search::launch_passC(int ka, int z0, int zn, long first_index, const long* desc) {
   dispatch_xh(Xh, [&](auto Lc) {
     constexpr int L = decltype(Lc)::value;
     constexpr int NL = passc_lines<L>();
     const long line0 = (long)z0 * Y, line1 = (long)(z0 + zn) * Y;
     const long nl = line1 - line0;
-    hipLaunchKernelGGL(k_passC<L>, dim3((unsigned)((nl + NL - 1) / NL)), dim3(NT_C), 0, s_, (const c32*)Q_, maxc_,
-                       argm_, tw_.f32(L), tw_.f32(X), line0, line1, (long)Z * Y * Xh, ka, (int)first_index, desc);
+    const unsigned blocks = (unsigned)((nl + NL - 1) / NL);
+    const int groups = passC_groups(ka), apb = (ka + groups - 1) / groups;
+    const int ng = (ka + apb - 1) / apb;
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(blocks, ng), dim3(NT_C), 0, s_, (const c32*)Q_, maxc_, argm_, tw_.f32(L),
+                         tw_.f32(X), line0, line1, (long)Z * Y * Xh, ka, (int)first_index, desc, apb, gmax_, garg_, N);
+    };
+    if (ng == 1) {
+      go(k_passC<L, false>);
+    } else {
+      go(k_passC<L, true>);
+      const long cnt = nl * X;
+      hipLaunchKernelGGL(k_merge_groups, dim3((unsigned)((cnt / 2 + NT - 1) / NT)), dim3(NT), 0, s_,
+                         (const float*)gmax_, (const uint8_t*)garg_, ng, N, line0 * X, cnt, (int)first_index, desc, ka,
+                         maxc_, argm_);
+    }
   });
   TOMHIP_CHECK(hipGetLastError());
 }
