@@ -32,8 +32,8 @@ COMMON = [
 # spell their fused multiply-adds out.
 _NOCONTRACT = ["-ffp-contract=off"]
 EXTRA = {"rotate.hip": _NOCONTRACT, "search.hip": _NOCONTRACT, "subtomo.hip": _NOCONTRACT,
-         "fused.hip": _NOCONTRACT, "util.hip": _NOCONTRACT, "picks.hip": _NOCONTRACT, "analysis.hip": _NOCONTRACT}
-SOURCES = ["search.hip", "fused.hip", "rotate.hip", "subtomo.hip", "picks.hip", "util.hip", "analysis.hip", "unet.hip", "pool.hip", "api.hip",
+         "fused.hip": _NOCONTRACT, "box.hip": _NOCONTRACT, "util.hip": _NOCONTRACT, "picks.hip": _NOCONTRACT, "analysis.hip": _NOCONTRACT}
+SOURCES = ["search.hip", "fused.hip", "box.hip", "rotate.hip", "subtomo.hip", "picks.hip", "util.hip", "analysis.hip", "unet.hip", "pool.hip", "api.hip",
            "em_io.cpp"]
 
 

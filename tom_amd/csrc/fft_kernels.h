@@ -46,11 +46,10 @@ __global__ __launch_bounds__(NT) void k_c2c_x(cpx<T>* data, long nlines, const c
 
 // In-place c2c along a strided axis. Element (col c, index e) of outer slice
 // o in batch b sits at data[b*bs + o*os + c + e*es]; grid = (col tiles,
-// outer, batch). If wmul is non-null the kernel runs forward, multiplies by
-// the real weight wmul[o*os + c + e*es], then runs the inverse (DIR ignored).
+// outer, batch).
 template <typename T, int L, int DIR>
 __global__ __launch_bounds__(NT) void k_c2c_strided(cpx<T>* data, int ncols, long es, long os, long bs,
-                                                    const cpx<T>* twg, const float* wmul) {
+                                                    const cpx<T>* twg) {
   constexpr int TW = strided_tw<T, L>();
   __shared__ cpx<T> buf[L * TW];
   __shared__ cpx<T> tw[L];
@@ -62,18 +61,7 @@ __global__ __launch_bounds__(NT) void k_c2c_strided(cpx<T>* data, int ncols, lon
     buf[i] = (c0 + c < ncols) ? base[c + e * es] : mk<T>(0, 0);
   }
   __syncthreads();
-  if (wmul == nullptr) {
-    lds_fft<T, L, TW, NT, DIR, Inter<TW>>(buf, tw);
-  } else {
-    lds_fft<T, L, TW, NT, -1, Inter<TW>>(buf, tw);
-    const float* wb = wmul + (long)blockIdx.y * os + c0;
-    for (int i = threadIdx.x; i < L * TW; i += NT) {
-      const int e = i / TW, c = i % TW;
-      if (c0 + c < ncols) buf[i] = scale(buf[i], (T)wb[c + e * es]);
-    }
-    __syncthreads();
-    lds_fft<T, L, TW, NT, 1, Inter<TW>>(buf, tw);
-  }
+  lds_fft<T, L, TW, NT, DIR, Inter<TW>>(buf, tw);
   for (int i = threadIdx.x; i < L * TW; i += NT) {
     const int e = i / TW, c = i % TW;
     if (c0 + c < ncols) base[c + e * es] = buf[i];
@@ -227,10 +215,10 @@ void fft3_c2c(cpx<T>* data, int X, int Y, int Z, int nb, int dir, Twiddles& tws,
     dim3 g((X + TW - 1) / TW, Z, nb);
     if (dir < 0)
       hipLaunchKernelGGL((k_c2c_strided<T, L, -1>), g, dim3(NT), 0, s, data, X, (long)X, XY, XYZ,
-                         tw_table<T>(tws, L), (const float*)nullptr);
+                         tw_table<T>(tws, L));
     else
       hipLaunchKernelGGL((k_c2c_strided<T, L, 1>), g, dim3(NT), 0, s, data, X, (long)X, XY, XYZ,
-                         tw_table<T>(tws, L), (const float*)nullptr);
+                         tw_table<T>(tws, L));
   });
   TOMHIP_CHECK(hipGetLastError());
   dispatch_len(Z, [&](auto Lc) {
@@ -239,10 +227,10 @@ void fft3_c2c(cpx<T>* data, int X, int Y, int Z, int nb, int dir, Twiddles& tws,
     dim3 g((X + TW - 1) / TW, Y, nb);
     if (dir < 0)
       hipLaunchKernelGGL((k_c2c_strided<T, L, -1>), g, dim3(NT), 0, s, data, X, XY, (long)X, XYZ,
-                         tw_table<T>(tws, L), (const float*)nullptr);
+                         tw_table<T>(tws, L));
     else
       hipLaunchKernelGGL((k_c2c_strided<T, L, 1>), g, dim3(NT), 0, s, data, X, XY, (long)X, XYZ,
-                         tw_table<T>(tws, L), (const float*)nullptr);
+                         tw_table<T>(tws, L));
   });
   TOMHIP_CHECK(hipGetLastError());
 }

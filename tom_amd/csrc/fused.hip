@@ -696,14 +696,10 @@ bool dispatch_y(int Y, F&& f) {
 
 namespace {
 const c32* z_list(Twiddles& tw, int Z) {
+  if (Z != 256) return line_list(tw, Z);
   return tw.list(Z, [&](std::vector<c32>& h) {
-    if (Z == 256) {
-      for (int w = 0; w < 16; ++w)
-        for (int k = 0; k < 16; ++k) h.push_back(Twiddles::root<float>(256, w * k));
-    } else {
-      line_tw_list(Z, h);
-    }
-    if (h.empty()) h.push_back(mk(1.f, 0.f));
+    for (int w = 0; w < 16; ++w)
+      for (int k = 0; k < 16; ++k) h.push_back(Twiddles::root<float>(256, w * k));
   });
 }
 const c32* bc_list(Twiddles& tw, int X, int Y) {

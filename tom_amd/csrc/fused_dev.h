@@ -57,6 +57,12 @@ inline void line_tw_list(int L, std::vector<c32>& out) {
         out.push_back(r < R ? Twiddles::root<float>(L, r * k * (L / (NS * R))) : mk(0.f, 0.f));
   }
 }
+inline const c32* line_list(Twiddles& tw, int L) {
+  return tw.list(L, [&](std::vector<c32>& h) {
+    line_tw_list(L, h);
+    if (h.empty()) h.push_back(mk(1.f, 0.f));
+  });
+}
 // the twiddles of a butterfly of stage S (k = j mod NS) on its inputs
 template <int L, int S, int DIR>
 __device__ __forceinline__ void line_twiddle(const c32* tw, int k, c32* t) {

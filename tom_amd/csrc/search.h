@@ -97,7 +97,6 @@ class Search {
   void release();
   void run_batch(const float* rm_dev, int ka, long first_index, const long* desc);
   void rotate_templates(const float* rm_dev, int count, float* tout, const long* desc, long rm_step);
-  void box_filter(int count, float* t, c32* work);
   bool use_fused(int ka) const;
   void launch_passA(int ka);
   void launch_passB(int ka, int z0, int zn);

@@ -37,6 +37,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "box.h"
 #include "dft16.h"
 #include "fft_io.h"
 #include "fused.h"
@@ -146,89 +147,6 @@ __global__ void k_fill_max(float* maxc, int32_t* argm, long n) {
 
 __global__ void k_square(const float* a, float* b, long n) {
   for (long i = (long)blockIdx.x * NT + threadIdx.x; i < n; i += (long)gridDim.x * NT) b[i] = a[i] * a[i];
-}
-
-// ---------------------------------------------------------------- box filter
-// real lines of L -> complex, forward FFT along x
-// Blocks never straddle two templates: every template's line j sits at the
-// same place in its block whatever the template's position in the batch, so a
-// template's filtered result does not depend on how the batch is grouped.
-__device__ __forceinline__ void box_block_lines(long lines_per_vol, int NL, long& l0, long& nl) {
-  const long nbt = (lines_per_vol + NL - 1) / NL;
-  const long a = blockIdx.x / nbt, b = blockIdx.x % nbt;
-  l0 = a * lines_per_vol + b * NL;
-  nl = (lines_per_vol - b * NL < NL) ? (lines_per_vol - b * NL) : NL;
-}
-
-template <int L>
-__global__ __launch_bounds__(NT) void k_box_x_fwd(const float* t, c32* out, long lines_per_vol, const c32* twg) {
-  constexpr int NL = contig_lines<float, L>();
-  __shared__ c32 buf[NL * L];
-  __shared__ c32 tw[L];
-  load_table<float, L, NT>(tw, twg);
-  long l0, nl;
-  box_block_lines(lines_per_vol, NL, l0, nl);
-  const int nval = (int)(nl * L);
-  for (int i = threadIdx.x; i < NL * L; i += NT) buf[i] = mk((i < nval) ? t[l0 * L + i] : 0.f, 0.f);
-  __syncthreads();
-  lds_fft<float, L, NL, NT, -1, Contig<L>>(buf, tw);
-  for (int i = threadIdx.x; i < nval; i += NT) out[l0 * L + i] = buf[i];
-}
-
-// inverse FFT along x, real part / n3, times mask -> float
-template <int L>
-__global__ __launch_bounds__(NT) void k_box_x_inv(const c32* in, float* t, const float* M, long lines_per_vol,
-                                                  float inv_n3, const c32* twg) {
-  constexpr int NL = contig_lines<float, L>();
-  __shared__ c32 buf[NL * L];
-  __shared__ c32 tw[L];
-  load_table<float, L, NT>(tw, twg);
-  long l0, nl;
-  box_block_lines(lines_per_vol, NL, l0, nl);
-  const int nval = (int)(nl * L);
-  for (int i = threadIdx.x; i < NL * L; i += NT) buf[i] = (i < nval) ? in[l0 * L + i] : mk(0.f, 0.f);
-  __syncthreads();
-  lds_fft<float, L, NL, NT, 1, Contig<L>>(buf, tw);
-  for (int i = threadIdx.x; i < nval; i += NT) {
-    const long g = l0 * L + i;
-    const long vox = ((g / L) % lines_per_vol) * L + (g % L);
-    t[g] = buf[i].x * inv_n3 * M[vox];
-  }
-}
-
-// Both in-plane transforms of one xy plane per block (square planes up to
-// 64 x 64): the plane sits in LDS with row pitch L + 1, x lines are rows,
-// y lines are columns. Same butterflies as the separate x and y passes, one
-// HBM round trip instead of two.
-template <int L>
-__global__ __launch_bounds__(NT) void k_box_xy_fwd(const float* t, c32* out, const c32* twg) {
-  constexpr int P = L + 1;
-  __shared__ c32 buf[L * P];
-  __shared__ c32 tw[L];
-  load_table<float, L, NT>(tw, twg);
-  const long base = (long)blockIdx.x * L * L;  // plane index over templates x planes
-  for (int i = threadIdx.x; i < L * L; i += NT) buf[(i / L) * P + i % L] = mk(t[base + i], 0.f);
-  __syncthreads();
-  lds_fft<float, L, L, NT, -1, Contig<P>>(buf, tw);
-  lds_fft<float, L, L, NT, -1, Inter<P>>(buf, tw);
-  for (int i = threadIdx.x; i < L * L; i += NT) out[base + i] = buf[(i / L) * P + i % L];
-}
-
-// inverse of the above, real part / n3, times mask -> float
-template <int L>
-__global__ __launch_bounds__(NT) void k_box_xy_inv(const c32* in, float* t, const float* M, int nz, float inv_n3,
-                                                   const c32* twg) {
-  constexpr int P = L + 1;
-  __shared__ c32 buf[L * P];
-  __shared__ c32 tw[L];
-  load_table<float, L, NT>(tw, twg);
-  const long base = (long)blockIdx.x * L * L;
-  const float* m = M + (long)(blockIdx.x % nz) * L * L;
-  for (int i = threadIdx.x; i < L * L; i += NT) buf[(i / L) * P + i % L] = in[base + i];
-  __syncthreads();
-  lds_fft<float, L, L, NT, 1, Inter<P>>(buf, tw);
-  lds_fft<float, L, L, NT, 1, Contig<P>>(buf, tw);
-  for (int i = threadIdx.x; i < L * L; i += NT) t[base + i] = buf[(i / L) * P + i % L].x * inv_n3 * m[i];
 }
 
 // ---------------------------------------------------------------- template fwd
@@ -1388,6 +1306,7 @@ void Search::capture_graph() {
   // twiddle tables are allocated on first use, which a capture does not allow
   for (int L : {nx, ny, nz, X, Y, Z, Xh}) (void)tw_.f32(L);
   if (use_fused(KA_)) fused_prepare(tw_, X, Y, Z);
+  if (wsh_) box_prepare(tw_, nx, ny, nz);
   hipGraph_t g = nullptr;
   TOMHIP_CHECK(hipStreamBeginCapture(s_, hipStreamCaptureModeThreadLocal));
   try {
@@ -1420,70 +1339,6 @@ void Search::rotate_templates(const float* rm_dev, int count, float* tout, const
   const float* rmask = nullptr;
   if (mode == MODE_FLCF) rmask = (wsh_ || !remask_) ? mask_ : mask_ + n3;
   launch_rotate(tmpl_, tout, rm_dev, count, rmask, nx, ny, nz, px, py, pz, n3, s_, desc, rm_step, tpairs_);
-}
-
-void Search::box_filter(int count, float* t, c32* work) {
-  // t <- M .* ifftn(fftn(t) .* W) per template (tom_os3_findTemplate.m:264-267
-  // followed by the masking inside tom_os3_corr)
-  const long n3 = (long)nx * ny * nz;
-  const long lpv = (long)ny * nz;  // x lines per template
-  const long XY = (long)nx * ny;
-  const bool plane = (nx == ny && nx <= 64);
-  if (plane) {
-    dispatch_len(nx, [&](auto Lc) {
-      constexpr int L = decltype(Lc)::value;
-      if constexpr (L <= 64)
-        hipLaunchKernelGGL(k_box_xy_fwd<L>, dim3((unsigned)(count * nz)), dim3(NT), 0, s_, (const float*)t, work,
-                           tw_.f32(L));
-    });
-    TOMHIP_CHECK(hipGetLastError());
-  } else {
-    dispatch_len(nx, [&](auto Lc) {
-      constexpr int L = decltype(Lc)::value;
-      constexpr int NL = contig_lines<float, L>();
-      hipLaunchKernelGGL(k_box_x_fwd<L>, dim3((unsigned)(count * ((lpv + NL - 1) / NL))), dim3(NT), 0, s_,
-                         (const float*)t, work, lpv, tw_.f32(L));
-    });
-    TOMHIP_CHECK(hipGetLastError());
-    dispatch_len(ny, [&](auto Lc) {
-      constexpr int L = decltype(Lc)::value;
-      constexpr int TW = strided_tw<float, L>();
-      hipLaunchKernelGGL((k_c2c_strided<float, L, -1>), dim3((nx + TW - 1) / TW, nz, count), dim3(NT), 0, s_, work,
-                         nx, (long)nx, XY, n3, tw_.f32(L), (const float*)nullptr);
-    });
-    TOMHIP_CHECK(hipGetLastError());
-  }
-  dispatch_len(nz, [&](auto Lc) {
-    constexpr int L = decltype(Lc)::value;
-    constexpr int TW = strided_tw<float, L>();
-    hipLaunchKernelGGL((k_c2c_strided<float, L, -1>), dim3((nx + TW - 1) / TW, ny, count), dim3(NT), 0, s_, work, nx,
-                       XY, (long)nx, n3, tw_.f32(L), (const float*)wsh_);
-  });
-  TOMHIP_CHECK(hipGetLastError());
-  if (plane) {
-    dispatch_len(nx, [&](auto Lc) {
-      constexpr int L = decltype(Lc)::value;
-      if constexpr (L <= 64)
-        hipLaunchKernelGGL(k_box_xy_inv<L>, dim3((unsigned)(count * nz)), dim3(NT), 0, s_, (const c32*)work, t,
-                           mask_, nz, (float)(1.0 / (double)n3), tw_.f32(L));
-    });
-    TOMHIP_CHECK(hipGetLastError());
-    return;
-  }
-  dispatch_len(ny, [&](auto Lc) {
-    constexpr int L = decltype(Lc)::value;
-    constexpr int TW = strided_tw<float, L>();
-    hipLaunchKernelGGL((k_c2c_strided<float, L, 1>), dim3((nx + TW - 1) / TW, nz, count), dim3(NT), 0, s_, work, nx,
-                       (long)nx, XY, n3, tw_.f32(L), (const float*)nullptr);
-  });
-  TOMHIP_CHECK(hipGetLastError());
-  dispatch_len(nx, [&](auto Lc) {
-    constexpr int L = decltype(Lc)::value;
-    constexpr int NL = contig_lines<float, L>();
-    hipLaunchKernelGGL(k_box_x_inv<L>, dim3((unsigned)(count * ((lpv + NL - 1) / NL))), dim3(NT), 0, s_,
-                       (const c32*)work, t, mask_, lpv, (float)(1.0 / (double)n3), tw_.f32(L));
-  });
-  TOMHIP_CHECK(hipGetLastError());
 }
 
 namespace {
@@ -1572,7 +1427,7 @@ bool Search::use_fused(int ka) const {
 void Search::run_batch(const float* rm_dev, int ka, long first_index, const long* desc) {
   const bool fused = use_fused(ka);
   timed(K_ROT, [&] { rotate_templates(rm_dev, ka, t1_, desc, 9L * ka); });
-  if (wsh_) timed(K_BOX, [&] { box_filter(ka, t1_, tbox_); });
+  if (wsh_) timed(K_BOX, [&] { box_filter(tw_, s_, ka, t1_, tbox_, wsh_, mask_, nx, ny, nz); });
 
   timed(K_TFWD, [&] {
     // the x-DFT rows go to the front of Q, which is free until pass A
@@ -1771,7 +1626,7 @@ void Search::refine(const float* volume, const float* rm_host, int G, int A, con
       const int a0 = c0 * KS;
       const int cnt = std::min(nb * KS, A - a0);
       rotate_templates(rm + 9L * a0 * G, cnt * G, tt, nullptr, 0);
-      if (wsh_) box_filter(cnt * G, tt, work);
+      if (wsh_) box_filter(tw_, s_, cnt * G, tt, work, wsh_, mask_, nx, ny, nz);
       hipLaunchKernelGGL(k_refine<KS>, dim3((unsigned)P, (unsigned)nb), dim3(NT_R), lds, s_, volume, X, Y, Z,
                          (const float*)tt, G, nx, ny, nz, sx, sy, sz, reinterpret_cast<const int4*>(cand_dev),
                          (const double*)mu_, (const double*)sig_, inv_m, mu_t, sig_t, a0, A,
