@@ -153,7 +153,7 @@ __global__ void k_square(const float* a, float* b, long n) {
 // x: direct DFT of the n non-zero samples of every template row for each
 // kx in [0, X/2], as register tiles of 4 rows x 4 frequencies (a row's
 // samples and a frequency's twiddles are each read once per tile and used 4
-// times). grid (nz, ka). Output Tx[a][uz][uy][kx], row pitch tx_pitch(Xh).
+// times). grid (nz, ka, groups of frequency tiles). Output Tx[a][uz][uy][kx], row pitch tx_pitch(Xh).
 // Summation order per output is ux ascending with fmaf, the twiddle index
 // kx (ux - hx) mod X advanced by kx per sample.
 constexpr int TXU = 4, TXK = 4;
@@ -174,7 +174,8 @@ __global__ __launch_bounds__(NT) void k_tmpl_xdft(const float* t2, c32* Tx, cons
   c32* dst = Tx + ((long)a * nz + uz) * ny * XP;
   // lanes run over row tiles first: the twiddles of a wave come from a few
   // frequency tiles (few LDS addresses), the padded rows from distinct banks
-  for (int q = threadIdx.x; q < nUT * nKT; q += NT) {
+  const int q0 = (threadIdx.x / 64 * gridDim.z + blockIdx.z) * 64 + threadIdx.x % 64;
+  for (int q = q0; q < nUT * nKT; q += gridDim.z * NT) {
     const int ut = q % nUT, kt = q / nUT;
     int kx[TXK], m[TXK];
 #pragma unroll
@@ -1432,7 +1433,11 @@ void Search::run_batch(const float* rm_dev, int ka, long first_index, const long
   timed(K_TFWD, [&] {
     // the x-DFT rows go to the front of Q, which is free until pass A
     c32* Tx = Tx_ ? Tx_ : Q_;
-    hipLaunchKernelGGL(k_tmpl_xdft, dim3(nz, ka), dim3(NT), 0, s_, (const float*)t1_, Tx, tw_.f32(X), X, nx, ny,
+    // few planes: their tiles over more blocks, a wave's or more each (24
+    // planes of 32 rows, X = 320, ka 4, 96 blocks and 480: 22.4 and 13.8 us)
+    const int tiles = (ny + TXU - 1) / TXU * ((tx_pitch(Xh) + TXK - 1) / TXK);
+    const int zg = std::max(1, std::min((tiles + 63) / 64, 512 / (nz * ka)));
+    hipLaunchKernelGGL(k_tmpl_xdft, dim3(nz, ka, zg), dim3(NT), 0, s_, (const float*)t1_, Tx, tw_.f32(X), X, nx, ny,
                        nz);
     dispatch_len(Y, [&](auto Lc) {
       constexpr int L = decltype(Lc)::value;
