@@ -27,27 +27,46 @@ __device__ double block_sum(double v, double* red) {
   return r;
 }
 
+// add(i, ld(i)) for the elements i = thread (mod NTB) in ascending order, 8
+// loads in flight: the sums below are one block's, so that their order is
+// fixed, and with a load at a time its threads wait for memory throughout
+// (48^3 voxels: k_norm_under_mask 104 us, now 57; a search of 256x256x128 with
+// one orientation 1,205 and 1,155).
+template <class LD, class ADD>
+__device__ __forceinline__ void block_elements(long n, const LD& ld, const ADD& add) {
+  constexpr int U = 8;
+  for (long i0 = threadIdx.x; i0 < n; i0 += U * NTB) {
+    decltype(ld(0L)) v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = ld(min(i0 + u * NTB, n - 1));
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i0 + u * NTB < n) add(i0 + u * NTB, v[u]);
+  }
+}
+
 // tom_norm(1e5*(T+1), 'mean0+1std') of tom_os3_findTemplate.m:157
 // (Sptrans/tom_norm.m:83-119; tom_dev population std, Analysis/tom_dev.m:55-60),
 // evaluated in FP64. Writes FP64 (for the statistics) and FP32 (the template
 // the search rotates).
-__global__ __launch_bounds__(NTB) void k_tnorm(const float* T, long n, double* out64, float* out32) {
+__global__ __launch_bounds__(NTB) void k_tnorm(const float* __restrict__ T, long n, double* out64, float* out32) {
   __shared__ double red[NTB];
+  auto ld = [&](long i) { return T[i]; };
   double s = 0;
-  for (long i = threadIdx.x; i < n; i += NTB) s += (1e5 * ((double)T[i] + 1.0)) * 2 + 100;
+  block_elements(n, ld, [&](long, float t) { s += (1e5 * ((double)t + 1.0)) * 2 + 100; });
   const double mea = block_sum(s, red) / (double)n;
   double q = 0;
-  for (long i = threadIdx.x; i < n; i += NTB) {
-    const double d = (1e5 * ((double)T[i] + 1.0)) * 2 + 100 - mea;
+  block_elements(n, ld, [&](long, float t) {
+    const double d = (1e5 * ((double)t + 1.0)) * 2 + 100 - mea;
     q += d * d;
-  }
+  });
   const double st = sqrt(block_sum(q, red) / (double)n);
-  for (long i = threadIdx.x; i < n; i += NTB) {
-    const double a = (1e5 * ((double)T[i] + 1.0)) * 2 + 100;
+  block_elements(n, ld, [&](long i, float t) {
+    const double a = (1e5 * ((double)t + 1.0)) * 2 + 100;
     const double v = (st != 0) ? (a - mea) / st : (a - mea);
     out64[i] = v;
     out32[i] = (float)v;
-  }
+  });
 }
 
 __global__ void k_to_c64(const double* a, c64* b, long n) {
@@ -65,27 +84,32 @@ __global__ void k_weight_real(c64* a, const float* wsh, long n) {
 
 // tom_os3_normUnderMask: mean over mask~=0 (and vol~=0), population std
 // (statistics/tom_os3_normUnderMask.m:1-8). tmp = Re(c)/scale.
-__global__ __launch_bounds__(NTB) void k_norm_under_mask(const c64* c, double scl, const float* M, long n,
-                                                         double* res) {
+__global__ __launch_bounds__(NTB) void k_norm_under_mask(const c64* __restrict__ c, double scl,
+                                                         const float* __restrict__ M, long n, double* res) {
   __shared__ double red[NTB];
+  struct El {
+    double c;
+    float m;
+  };
+  auto ld = [&](long i) { return El{c[i].x, M[i]}; };
   double cnt = 0, s = 0;
-  for (long i = threadIdx.x; i < n; i += NTB) {
-    if (M[i] != 0.f) {
-      const double v = c[i].x * scl;
+  block_elements(n, ld, [&](long, const El& e) {
+    if (e.m != 0.f) {
+      const double v = e.c * scl;
       cnt += 1;
       s += (v != 0) ? v : 0;
     }
-  }
+  });
   cnt = block_sum(cnt, red);
   s = block_sum(s, red);
   const double mea = s / cnt;
   double q = 0;
-  for (long i = threadIdx.x; i < n; i += NTB) {
-    if (M[i] != 0.f) {
-      const double d = c[i].x * scl - mea;
+  block_elements(n, ld, [&](long, const El& e) {
+    if (e.m != 0.f) {
+      const double d = e.c * scl - mea;
       q += d * d;
     }
-  }
+  });
   q = block_sum(q, red);
   if (threadIdx.x == 0) {
     res[0] = mea;
