@@ -88,9 +88,13 @@ void put(const void* p, hipStream_t s, bool idle) noexcept {
   const int device = it->second.first;
   Block b = it->second.second;
   S.used.erase(it);
-  b.idle = idle;
+  // a stream that has run dry needs no event: most calls wait for their results
+  // before they give their workspaces back (with an event each, a refinement
+  // of 7 candidates took 646 us for 605, 16 subtomograms of 32^3 540 for 415)
+  b.idle = idle || hipStreamQuery(s) == hipSuccess;
   b.stream = s;
-  if (!idle) {
+  if (!b.idle) {
+    (void)hipGetLastError();  // not ready
     if (!b.ev && hipEventCreateWithFlags(&b.ev, hipEventDisableTiming) != hipSuccess) b.ev = nullptr;
     if (!b.ev || hipEventRecord(b.ev, s) != hipSuccess) {
       (void)hipGetLastError();
