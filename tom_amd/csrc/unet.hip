@@ -927,7 +927,7 @@ __global__ __launch_bounds__(NTU) void k_up_bwd(const float* __restrict__ dY, in
 //
 // A wave takes 64 voxels: a lane each for channel 0, then all lanes together
 // for each voxel with a bin or offset target (a channel a lane: coalesced,
-// and the softmax sums are shuffles). The 64 rows are put together in LDS, where
+// the softmax's sum through scalar registers). The 64 rows are put together in LDS, where
 // they are zero but for the voxels that wrote to them, and stored in 16-byte
 // units. Bound by its writes, 160 bytes a voxel: 96^3 voxels 500 us (one
 // voxel a thread, FP32 rows) + 139 us (conversion and sums) -> 75 us.
@@ -974,8 +974,11 @@ __global__ __launch_bounds__(NTU) void k_loss(const float* __restrict__ logits, 
         float mx = fmaxf(x0, x1);
         for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
         const float e0 = lane < nbin ? expf(x0 - mx) : 0.f, e1 = lane + 64 < nbin ? expf(x1 - mx) : 0.f;
-        float se = e0 + e1;
-        for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
+        // in channel order: another order moves the last bit, and with it now
+        // and then a bf16 result
+        float se = 0.f;
+        for (int c = 0; c < nbin; ++c)
+          se += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c < 64 ? e0 : e1), c & 63));
         if (br < 64 ? lane == br : lane + 64 == br) l2 += -((br < 64 ? x0 : x1) - mx - logf(se));
         if (lane < nbin) g[0] = (e0 / se - (lane == br ? 1.f : 0.f)) * inv_npos;
         if (lane + 64 < nbin) g[1] = (e1 / se - (lane + 64 == br ? 1.f : 0.f)) * inv_npos;
