@@ -38,8 +38,8 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch group measured with rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE (fetch scaled x2.000, write x1.000 by a 1 GiB device copy in the
 # same runs); profiles/flcf_c2_hbm_traffic.md has the commands and counts.
-# (config, batch) -> pass -> bytes
-MEASURED_TRAFFIC = {}
+# (config, batch) -> pass -> bytes; passA is k_fused_a, passC k_fused_bc
+MEASURED_TRAFFIC = {("c2", 16): {"passA": 5.6902e+09, "passC": 4.9826e+09}}
 
 def log(msg):
     print(msg, file=sys.stderr, flush=True)
