@@ -44,6 +44,7 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 constexpr int NTU = 256;
+constexpr int LCH = 80;  // channels of the head
 
 struct Dims {
   int D, H, W;
@@ -125,98 +126,8 @@ __global__ __launch_bounds__(NTU) void k_conv(const uint16_t* __restrict__ X, in
   }
 }
 
-// LDS-tiled convolution for the full-resolution layers: a block stages its
-// input tile of (16 + 2) x (4 + 2) x (TZ + 2) voxels x Cin channels (zero
-// outside the volume) in LDS once; wave w owns row y0 + w of the tile and its
-// TZ planes of 16 x voxels, so every A fragment is an LDS read and one weight
-// fragment (global, cache-resident) feeds TZ x CT MFMAs. Channel pitch Cin + 4
-// in LDS keeps 8-byte fragments aligned and spreads the voxel rows over banks.
+// voxels of a 3x3x3 block's tile in x and y
 constexpr int CTX = 16, CTY = 4;
-template <int CT, int CTZ>
-__global__ __launch_bounds__(NTU) void k_conv_t(const uint16_t* __restrict__ X, int xs, int xo, int Cin, Dims d,
-                                                const uint16_t* __restrict__ Wt, const float* __restrict__ bias,
-                                                int taps, int relu, uint16_t* Yb, int ys, int yo, float* Yf) {
-  extern __shared__ uint16_t tile[];
-  constexpr int Cout = 16 * CT;
-  constexpr int SX = CTX + 2, SY = CTY + 2, SZ = CTZ + 2;
-  const int CP = Cin + 4;
-  const int nbx = (d.W + CTX - 1) / CTX, nby = (d.H + CTY - 1) / CTY;
-  const int x0 = (blockIdx.x % nbx) * CTX, y0 = ((blockIdx.x / nbx) % nby) * CTY, z0 = (blockIdx.x / (nbx * nby)) * CTZ;
-  const int nch = Cin / 4;
-  const int total = SX * SY * SZ * nch;
-  for (int i = threadIdx.x; i < total; i += NTU) {
-    const int ch = i % nch, v = i / nch;
-    const int gx = x0 + v % SX - 1, gy = y0 + (v / SX) % SY - 1, gz = z0 + v / (SX * SY) - 1;
-    uint2 val = make_uint2(0u, 0u);
-    if (gx >= 0 && gx < d.W && gy >= 0 && gy < d.H && gz >= 0 && gz < d.D)
-      val = *reinterpret_cast<const uint2*>(X + (((long)gz * d.H + gy) * d.W + gx) * xs + xo + ch * 4);
-    *reinterpret_cast<uint2*>(tile + (long)v * CP + ch * 4) = val;
-  }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int row = lane & 15, kq = lane >> 4;
-  const int y = y0 + wv;
-  if (y >= d.H) return;  // no barrier follows
-  f32x4 acc[CTZ][CT];
-#pragma unroll
-  for (int zp = 0; zp < CTZ; ++zp)
-#pragma unroll
-    for (int j = 0; j < CT; ++j) acc[zp][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int KS = Cin / 16;
-  for (int t = 0; t < taps; ++t) {
-    int dz = 0, dy = 0, dx = 0;
-    if (taps == 27) {
-      dz = t / 9 - 1;
-      dy = (t / 3) % 3 - 1;
-      dx = t % 3 - 1;
-    }
-    const uint16_t* wp = Wt + ((long)t * Cout + row) * Cin;
-    const uint16_t* ap = tile + (long)(((dz + 1) * SY + (wv + dy + 1)) * SX + (row + dx + 1)) * CP;
-    for (int ks = 0; ks < KS; ++ks) {
-      const int c = ks * 16 + kq * 4;
-      bf16x4 b[CT];
-#pragma unroll
-      for (int j = 0; j < CT; ++j) {
-        const uint2 rw = *reinterpret_cast<const uint2*>(wp + (long)j * 16 * Cin + c);
-        b[j][0] = (short)(rw.x & 0xffff);
-        b[j][1] = (short)(rw.x >> 16);
-        b[j][2] = (short)(rw.y & 0xffff);
-        b[j][3] = (short)(rw.y >> 16);
-      }
-#pragma unroll
-      for (int zp = 0; zp < CTZ; ++zp) {
-        const uint2 raw = *reinterpret_cast<const uint2*>(ap + (long)zp * SY * SX * CP + c);
-        bf16x4 a;
-        a[0] = (short)(raw.x & 0xffff);
-        a[1] = (short)(raw.x >> 16);
-        a[2] = (short)(raw.y & 0xffff);
-        a[3] = (short)(raw.y >> 16);
-#pragma unroll
-        for (int j = 0; j < CT; ++j) acc[zp][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[j], acc[zp][j], 0, 0, 0);
-      }
-    }
-  }
-#pragma unroll
-  for (int zp = 0; zp < CTZ; ++zp) {
-    const int z = z0 + zp;
-    if (z >= d.D) continue;
-#pragma unroll
-    for (int j = 0; j < CT; ++j) {
-      const int co = j * 16 + row;
-      const float bb = bias ? bias[co] : 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int x = x0 + 4 * kq + i;
-        if (x >= d.W) continue;
-        float v = acc[zp][j][i] + bb;
-        if (relu) v = fmaxf(v, 0.f);
-        const long vox = ((long)z * d.H + y) * d.W + x;
-        if (Yb) Yb[vox * ys + yo + co] = f2bf(v);
-        if (Yf) Yf[vox * Cout + co] = v;
-      }
-    }
-  }
-}
 
 // 3x3x3 convolution on v_mfma_f32_16x16x32_bf16 with the output as
 // D[cout][voxel] = W[cout][k] X[k][voxel]. K runs over chunks of CC input
@@ -471,6 +382,50 @@ __global__ __launch_bounds__(NTU) void k_conv_in(InWin in, Dims d, const uint16_
   }
 }
 
+// 1x1x1 convolution of 16 channels (rows of xs) to 16 CT FP32 channels. A wave
+// takes 16 voxels: D[cout][voxel] = W X, so a lane holds four neighbouring
+// channels of a voxel; the 16 rows go through LDS and leave as whole 16-byte
+// lines. Bound by its writes, 64 CT bytes a voxel: 96^3, 80 channels, 153 us
+// in LDS tiles of the input (stores of 4 bytes a lane, 64 of every 320) and 58
+// now.
+template <int CT>
+__global__ __launch_bounds__(NTU) void k_head_logits(const uint16_t* __restrict__ X, int xs, int xo, int V,
+                                                     const uint16_t* __restrict__ Wt, const float* __restrict__ bias,
+                                                     float* __restrict__ Y) {
+  constexpr int C = 16 * CT, P = C + 4;
+  __shared__ float4 tile[NTU / 64][16 * P / 4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int col = lane & 15, kq = lane >> 4;
+  bf16x4 w[CT];
+  float4 b[CT];
+#pragma unroll
+  for (int j = 0; j < CT; ++j) {
+    w[j] = __builtin_bit_cast(bf16x4, *reinterpret_cast<const uint2*>(Wt + (16 * j + col) * 16 + 4 * kq));
+    b[j] = *reinterpret_cast<const float4*>(bias + 16 * j + 4 * kq);
+  }
+  for (int v0 = (blockIdx.x * (NTU / 64) + wv) * 16; v0 < V; v0 += gridDim.x * (NTU / 64) * 16) {
+    const long v = min(v0 + col, V - 1);
+    const bf16x4 x = __builtin_bit_cast(bf16x4, *reinterpret_cast<const uint2*>(X + v * xs + xo + 4 * kq));
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      f32x4 a = {0.f, 0.f, 0.f, 0.f};
+      a = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w[j], x, a, 0, 0, 0);
+      tile[wv][col * (P / 4) + 4 * j + kq] = make_float4(a[0] + b[j].x, a[1] + b[j].y, a[2] + b[j].z, a[3] + b[j].w);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    float4* out = reinterpret_cast<float4*>(Y + (long)v0 * C);
+    const int n = min(16, V - v0) * (C / 4);
+#pragma unroll
+    for (int k = 0; k < CT; ++k) {
+      const int i = k * 64 + lane;
+      if (i < n) out[i] = tile[wv][i / (C / 4) * (P / 4) + i % (C / 4)];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 // Fragment order of 3x3x3 weights Wt [27][Cout][Cin] for k_conv3:
 // Wm[q][g][dz][j][lane][e] = Wt[9 dz + qi][16 j + (lane & 15)][q CC + c] with
 // k = 8 (lane >> 4) + e, qi = g NQ + k / CC, c = k % CC (0 where qi >= 9).
@@ -525,11 +480,10 @@ __device__ __forceinline__ bf16x4 quad_transpose(uint2 r, int i) {
   return __builtin_bit_cast(bf16x4, make_uint2(__builtin_amdgcn_perm(oa, a, sel), __builtin_amdgcn_perm(ob, b, sel)));
 }
 
-template <int TAPS>
 __global__ __launch_bounds__(64 * DWN) void k_conv_dw(const uint16_t* __restrict__ X, int xs, int xo, long xq, int Cin,
                                                       const uint16_t* __restrict__ dY, int Cout, Dims d,
                                                       float* part) {
-  constexpr int N = TAPS == 27 ? 3 : 1, R = N / 2;  // taps per axis, reach
+  constexpr int TAPS = 27, N = 3, R = 1;  // taps, taps per axis, reach
   __shared__ f32x4 red[DWN / 2][9][64];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i4 = lane & 3, cg = (lane >> 2) & 3, kq = lane >> 4;
@@ -576,23 +530,17 @@ __global__ __launch_bounds__(64 * DWN) void k_conv_dw(const uint16_t* __restrict
     };
     uint2 rx[N], ry[N], r0[N], r1[N];
     bf16x4 fx[N], fy[N][N];  // fy[dy]: the rows y + R .. y - R of dY, by plane
-    if (R) {
-      yrow(y0 - 1, r0);
-      yrow(y0, r1);
-    }
+    yrow(y0 - 1, r0);
+    yrow(y0, r1);
     yrow(y0 + R, ry);
     xrow(y0, rx);
-    if constexpr (R) {
-      yfrag(y0 - 1, r0, fy[1]);
-      yfrag(y0, r1, fy[0]);
-    }
+    yfrag(y0 - 1, r0, fy[1]);
+    yfrag(y0, r1, fy[0]);
     for (int y = y0; y < y1; ++y) {
-      if constexpr (R) {
 #pragma unroll
-        for (int k = 0; k < N; ++k) {
-          fy[2][k] = fy[1][k];
-          fy[1][k] = fy[0][k];
-        }
+      for (int k = 0; k < N; ++k) {
+        fy[2][k] = fy[1][k];
+        fy[1][k] = fy[0][k];
       }
       yfrag(y + R, ry, fy[0]);
 #pragma unroll
@@ -625,6 +573,60 @@ __global__ __launch_bounds__(64 * DWN) void k_conv_dw(const uint16_t* __restrict
     f32x4* o = reinterpret_cast<f32x4*>(part) + ((long)blockIdx.y * gridDim.x + blockIdx.x) * TAPS * 64 + lane;
 #pragma unroll
     for (int t = 0; t < TAPS; ++t) o[t * 64] = acc[t];
+  }
+}
+
+// Weight gradient of the 1x1x1 head, 16 channels of X (rows of xs) to 16 CT of
+// dY: part[j][block][...] for its CT pairs. K is the flat voxels, a wave takes
+// groups of 16 of them and all CT channel groups, so that rows are read whole
+// and once: 96^3, 80 channels, 101 us with a pair a block (32 of every 160
+// bytes, five times X) and 28 now.
+template <int CT>
+__global__ __launch_bounds__(64 * DWN) void k_head_dw(const uint16_t* __restrict__ X, int xs, int xo,
+                                                      const uint16_t* __restrict__ dY, int V, float* part) {
+  __shared__ f32x4 red[DWN / 2][CT][64];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i4 = lane & 3, cg = (lane >> 2) & 3, kq = lane >> 4;
+  const int groups = (V + 15) / 16, step = gridDim.x * DWN;
+  f32x4 acc[CT];
+#pragma unroll
+  for (int j = 0; j < CT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  uint2 rx, ry[CT];
+  auto load = [&](int g) {
+    const long v = min(g * 16 + 4 * kq + i4, V - 1);
+    rx = *reinterpret_cast<const uint2*>(X + v * xs + xo + 4 * cg);
+#pragma unroll
+    for (int j = 0; j < CT; ++j) ry[j] = *reinterpret_cast<const uint2*>(dY + v * (16 * CT) + 16 * j + 4 * cg);
+  };
+  int g = blockIdx.x * DWN + wv;
+  if (g < groups) load(g);
+  for (; g < groups; g += step) {
+    const bool in = g * 16 + 4 * kq + i4 < V;
+    const bf16x4 fx = quad_transpose(make_uint2(in ? rx.x : 0u, in ? rx.y : 0u), i4);
+    bf16x4 fy[CT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j) fy[j] = quad_transpose(make_uint2(in ? ry[j].x : 0u, in ? ry[j].y : 0u), i4);
+    if (g + step < groups) load(g + step);
+#pragma unroll
+    for (int j = 0; j < CT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fy[j], fx, acc[j], 0, 0, 0);
+  }
+#pragma unroll
+  for (int h = DWN / 2; h; h /= 2) {
+    if (wv >= h && wv < 2 * h) {
+#pragma unroll
+      for (int j = 0; j < CT; ++j) red[wv - h][j][lane] = acc[j];
+    }
+    __syncthreads();
+    if (wv < h) {
+#pragma unroll
+      for (int j = 0; j < CT; ++j) acc[j] += red[wv][j][lane];
+    }
+    __syncthreads();
+  }
+  if (wv == 0) {
+    f32x4* o = reinterpret_cast<f32x4*>(part) + (long)blockIdx.x * 64 + lane;
+#pragma unroll
+    for (int j = 0; j < CT; ++j) o[(long)j * gridDim.x * 64] = acc[j];
   }
 }
 
@@ -711,10 +713,17 @@ __global__ __launch_bounds__(NTU) void k_relu_bwd(PostGrad P, const uint16_t* __
 #pragma unroll
   for (int k = 0; k < 4; ++k) red[t][k] = sum[k];
   __syncthreads();
+  // four of a channel's 4 NTU / C sums a thread, then the rest by its first
+  const int c = t % C, q = t / C, np = NTU / C;
+  float a = 0.f;
+#pragma unroll
+  for (int m = 0; m < 4; ++m) a += red[c / 4 + C4 * (q + np * m)][c % 4];
+  __syncthreads();
+  float* r1 = &red[0][0];
+  r1[t] = a;
+  __syncthreads();
   if (t < C) {
-    const int cg = t / 4, k = t % 4;
-    float a = 0.f;
-    for (int r = cg; r < per * C4; r += C4) a += red[r][k];
+    for (int m = 1; m < np; ++m) a += r1[t + C * m];
     atomicAdd(&dbias[t], a);
   }
 }
@@ -930,8 +939,8 @@ __global__ __launch_bounds__(NTU) void k_up_bwd(const float* __restrict__ dY, in
 // the softmax's sum through scalar registers). The 64 rows are put together in LDS, where
 // they are zero but for the voxels that wrote to them, and stored in 16-byte
 // units. Bound by its writes, 160 bytes a voxel: 96^3 voxels 500 us (one
-// voxel a thread, FP32 rows) + 139 us (conversion and sums) -> 75 us.
-constexpr int LCH = 80;
+// voxel a thread, FP32 rows) + 139 us (conversion and sums) -> 116 us, 40 of
+// them the softmax's sums in channel order where a voxel in 20 has a target.
 __global__ __launch_bounds__(NTU) void k_loss(const float* __restrict__ logits, int nbin,
                                               const float* __restrict__ tprob, const int32_t* __restrict__ tbin,
                                               const float* __restrict__ toff, long V, float wpos, float inv_v,
@@ -1375,73 +1384,53 @@ void conv_forward(const uint16_t* X, int xs, int xo, long xq, int Cin, int D, in
     return;
   }
   TOMHIP_REQUIRE(xq == 0, ERR_UNSUPPORTED, "conv: 1x1x1 needs an interleaved input");
-  // LDS tile of (CTZ + 2) planes; 4 planes per wave when the tile fits in
-  // 64 KB, else 2
-  auto lds_for = [&](int tz) { return sizeof(uint16_t) * (CTX + 2) * (CTY + 2) * (tz + 2) * (size_t)(Cin + 4); };
-  const int tz = lds_for(4) <= 65536 ? 4 : 2;
-  const size_t lds = lds_for(tz);
-  if (lds <= 65536) {
-    dim3 g((unsigned)(((W + CTX - 1) / CTX) * ((H + CTY - 1) / CTY) * ((D + tz - 1) / tz)));
-    auto go = [&](auto TZc) {
-      constexpr int TZ = decltype(TZc)::value;
-      switch (Cout / 16) {
+  if (Cin == 16 && Cout == LCH && Yf && !Yb && !relu && bias) {  // the head
+    const int V = (int)d.V();
+    hipLaunchKernelGGL(k_head_logits<LCH / 16>, dim3(std::min((V + 63) / 64, 2048)), dim3(NTU), 0, s, X, xs, xo, V, Wt,
+                       bias, Yf);
+    TOMHIP_CHECK(hipGetLastError());
+    return;
+  }
+  dim3 g((unsigned)(((W + 15) / 16) * ((H + 3) / 4) * D));
+  switch (Cout / 16) {
 #define TOMHIP_CONV_CASE(ct)                                                                                     \
   case ct:                                                                                                    \
-    hipLaunchKernelGGL((k_conv_t<ct, TZ>), g, dim3(NTU), lds, s, X, xs, xo, Cin, d, Wt, bias, taps, relu, Yb, ys, \
-                       yo, Yf);                                                                               \
-    break;
-        TOMHIP_CONV_CASE(1)
-        TOMHIP_CONV_CASE(2)
-        TOMHIP_CONV_CASE(3)
-        TOMHIP_CONV_CASE(4)
-        TOMHIP_CONV_CASE(5)
-        TOMHIP_CONV_CASE(6)
+  hipLaunchKernelGGL(k_conv<ct>, g, dim3(NTU), 0, s, X, xs, xo, Cin, d, Wt, bias, taps, relu, Yb, ys, yo, Yf); \
+  break;
+    TOMHIP_CONV_CASE(1)
+    TOMHIP_CONV_CASE(2)
+    TOMHIP_CONV_CASE(3)
+    TOMHIP_CONV_CASE(4)
+    TOMHIP_CONV_CASE(5)
+    TOMHIP_CONV_CASE(6)
 #undef TOMHIP_CONV_CASE
-      }
-    };
-    if (tz == 4)
-      go(std::integral_constant<int, 4>{});
-    else
-      go(std::integral_constant<int, 2>{});
-  } else {
-    dim3 g((unsigned)(((W + 15) / 16) * ((H + 3) / 4) * D));
-    switch (Cout / 16) {
-#define TOMHIP_CONV_CASE(ct)                                                                                     \
-  case ct:                                                                                                    \
-    hipLaunchKernelGGL(k_conv<ct>, g, dim3(NTU), 0, s, X, xs, xo, Cin, d, Wt, bias, taps, relu, Yb, ys, yo, Yf); \
-    break;
-      TOMHIP_CONV_CASE(1)
-      TOMHIP_CONV_CASE(2)
-      TOMHIP_CONV_CASE(3)
-      TOMHIP_CONV_CASE(4)
-      TOMHIP_CONV_CASE(5)
-      TOMHIP_CONV_CASE(6)
-#undef TOMHIP_CONV_CASE
-    }
   }
   TOMHIP_CHECK(hipGetLastError());
 }
 
 // Blocks of a weight gradient's pair of channel groups: one for each CU over
-// all pairs, as far as there are units of work.
-static int dw_blocks(int Cin, int Cout, int D, int H, int W) {
+// all pairs (1x1x1: over all voxels), as far as there are units of work.
+static int dw_blocks(int Cin, int Cout, int D, int H, int W, int taps) {
+  if (taps == 1) return (int)std::min(((long)D * H * W + 16 * DWN - 1) / (16 * DWN), (long)DWBLK);
   const long units = (long)D * ((H + DWY - 1) / DWY) * ((W + 15) / 16);
   const int pairs = (Cin / 16) * (Cout / 16);
   return (int)std::min((units + DWN - 1) / DWN, (long)std::max(1, DWBLK / pairs));
 }
 long conv_weight_grad_elems(int Cin, int Cout, int D, int H, int W, int taps) {
-  return (long)(Cin / 16) * (Cout / 16) * dw_blocks(Cin, Cout, D, H, W) * taps * 256;
+  return (long)(Cin / 16) * (Cout / 16) * dw_blocks(Cin, Cout, D, H, W, taps) * taps * 256;
 }
 
 void conv_weight_grad(const uint16_t* X, int xs, int xo, long xq, int Cin, const uint16_t* dY, int Cout, int D, int H,
                       int W, int taps, float* dW, float* part, hipStream_t s) {
   Dims d{D, H, W};
   const unsigned pairs = (unsigned)((Cout / 16) * (Cin / 16));
-  const int nb = dw_blocks(Cin, Cout, D, H, W);
-  if (taps == 27)
-    hipLaunchKernelGGL(k_conv_dw<27>, dim3(nb, pairs), dim3(64 * DWN), 0, s, X, xs, xo, xq, Cin, dY, Cout, d, part);
-  else
-    hipLaunchKernelGGL(k_conv_dw<1>, dim3(nb, pairs), dim3(64 * DWN), 0, s, X, xs, xo, xq, Cin, dY, Cout, d, part);
+  const int nb = dw_blocks(Cin, Cout, D, H, W, taps);
+  if (taps == 27) {
+    hipLaunchKernelGGL(k_conv_dw, dim3(nb, pairs), dim3(64 * DWN), 0, s, X, xs, xo, xq, Cin, dY, Cout, d, part);
+  } else {
+    TOMHIP_REQUIRE(Cin == 16 && Cout == LCH && xq == 0, ERR_UNSUPPORTED, "1x1x1 weight gradient: the head's only");
+    hipLaunchKernelGGL(k_head_dw<LCH / 16>, dim3(nb), dim3(64 * DWN), 0, s, X, xs, xo, dY, (int)d.V(), part);
+  }
   hipLaunchKernelGGL(k_dw_sum, dim3(taps * 4, pairs), dim3(1024), 0, s, (const float*)part, nb, taps, Cin, Cout, dW);
   TOMHIP_CHECK(hipGetLastError());
 }
