@@ -15,7 +15,15 @@ void work_get(T** p, size_t bytes, hipStream_t s) {
 // Gives a workspace back; what is queued on s so far may still use it. Null
 // is ignored.
 void work_put(const void* p, hipStream_t s) noexcept;
-// The same for a workspace that nothing queued anywhere uses.
+// Gives *p back and takes a workspace of `bytes` in its place. Where that
+// fails *p is null: no pointer to a workspace that has been given back stays.
+template <typename T>
+void work_renew(T** p, size_t bytes, hipStream_t s) {
+  work_put(*p, s);
+  *p = nullptr;
+  work_get(p, bytes, s);
+}
+// work_put for a workspace that nothing queued anywhere uses.
 void work_put_idle(const void* p) noexcept;
 
 // Contexts of a device, counted: the last one to go frees what is kept.

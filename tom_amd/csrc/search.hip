@@ -1280,10 +1280,10 @@ void Search::run(const float* rm_host, long count, long first_index) {
   if (count <= 0) return;
   TOMHIP_REQUIRE(first_index >= 0 && first_index + count <= INT32_MAX, ERR_WRONG_INPUT, "angle index range");
   if (count > rm_cap_) {
-    work_put(rm_, s_);
-    work_get(&rm_, sizeof(float) * 9 * count, s_);
+    drop_graph();  // it reads the list that goes
+    rm_cap_ = 0;
+    work_renew(&rm_, sizeof(float) * 9 * count, s_);
     rm_cap_ = count;
-    drop_graph();  // captured pointers changed
   }
   TOMHIP_CHECK(hipMemcpyAsync(rm_, rm_host, sizeof(float) * 9 * count, hipMemcpyHostToDevice, s_));
   const long nfull = count / KA_;
