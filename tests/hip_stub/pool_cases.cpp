@@ -40,11 +40,54 @@ static int renew() {
   return 0;
 }
 
+// A block whose stream has work queued is waited for also where the next call
+// names the same handle: a handle is not a stream (a destroyed stream's may
+// come back as another one's).
+static int same_handle() {
+  FakeStream s;
+  work_device_up(0);
+  void* p = work_get(4096, &s);
+  ++s.queued;
+  work_put(p, &s);
+  s.done = 0;
+  HOLDS(work_get(4096, &s) == p);
+  HOLDS(fake().waits == 1);
+  // once the stream has run dry nothing is waited for
+  s.done = s.queued;
+  work_put(p, &s);
+  HOLDS(work_get(4096, &s) == p);
+  HOLDS(fake().waits == 1);
+  work_put(p, &s);
+  work_device_down(0);
+  HOLDS(fake().live.empty());
+  return 0;
+}
+
+// hipStreamPerThread is another stream in every thread, so neither a query nor
+// an event of the thread that gives a block back says when the work of another
+// one has left it: such a block goes to the driver, which waits for the device.
+static int per_thread() {
+  work_device_up(0);
+  void* p = work_get(4096, hipStreamPerThread);
+  work_put(p, hipStreamPerThread);  // dry in this thread
+  HOLDS(fake().frees == 1);
+  FakeStream s;
+  p = work_get(8192, &s);
+  ++s.queued;
+  work_put(p, &s);
+  HOLDS(work_get(8192, hipStreamPerThread) == p && fake().waits == 1);
+  work_put(p, hipStreamPerThread);
+  HOLDS(fake().frees == 2);
+  work_device_down(0);
+  HOLDS(fake().live.empty() && fake().freed_twice.empty());
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*f)();
-  } cases[] = {{"renew", renew}};
+  } cases[] = {{"renew", renew}, {"same_handle", same_handle}, {"per_thread", per_thread}};
   for (auto& c : cases)
     if (argc == 2 && !strcmp(argv[1], c.name)) return c.f();
   printf("no such case\n");

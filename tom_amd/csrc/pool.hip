@@ -4,10 +4,11 @@
 // all, and gave them back to the driver at its end: 3 to 24 ms of hipMalloc
 // and hipFree (it differs from machine to machine) around 0.95 ms of kernels.
 // Here a freed workspace waits for the next request of its size. It carries
-// an event recorded on the stream that used it last, which a request for
-// another stream waits for, so calls on several streams and threads may share
-// the pool. At most kKeep bytes wait per device, oldest out first; all of it
-// goes when an allocation fails or the device's last context is destroyed.
+// an event recorded on the stream that used it last, which the next request
+// waits for whatever stream it names (equal handles may be different streams),
+// so calls on several streams and threads may share the pool. At most kKeep
+// bytes wait per device, oldest out first; all of it goes when an allocation
+// fails or the device's last context is destroyed.
 #include <map>
 #include <mutex>
 #include <vector>
@@ -25,8 +26,7 @@ struct Block {
   void* p = nullptr;
   size_t size = 0;
   hipEvent_t ev = nullptr;
-  hipStream_t stream = nullptr;  // of the last use
-  bool idle = true;              // nothing queued uses it
+  bool idle = true;  // nothing queued uses it
 };
 
 struct Device {
@@ -88,17 +88,22 @@ void put(const void* p, hipStream_t s, bool idle) noexcept {
   const int device = it->second.first;
   Block b = it->second.second;
   S.used.erase(it);
+  // the per-thread handle names another stream in each thread: what this
+  // thread's has done says nothing of the work another thread queued
+  if (!idle && s == hipStreamPerThread) {
+    drop(b);  // hipFree waits for the device
+    return;
+  }
   // a stream that has run dry needs no event: most calls wait for their results
   // before they give their workspaces back (with an event each, a refinement
   // of 7 candidates took 646 us for 605, 16 subtomograms of 32^3 540 for 415)
   b.idle = idle || hipStreamQuery(s) == hipSuccess;
-  b.stream = s;
   if (!b.idle) {
     (void)hipGetLastError();  // not ready
     if (!b.ev && hipEventCreateWithFlags(&b.ev, hipEventDisableTiming) != hipSuccess) b.ev = nullptr;
     if (!b.ev || hipEventRecord(b.ev, s) != hipSuccess) {
       (void)hipGetLastError();
-      drop(b);  // hipFree waits for the device
+      drop(b);
       return;
     }
   }
@@ -119,7 +124,7 @@ void* work_get(size_t bytes, hipStream_t s) {
   std::lock_guard<std::mutex> g(S.mu);
   Device& d = S.dev[device];
   // the smallest kept block that fits without wasting more than a quarter
-  // (or a page), one of this stream first
+  // (or a page), one that nothing uses first
   int best = -1;
   for (int i = 0; i < (int)d.kept.size(); ++i) {
     const Block& b = d.kept[i];
@@ -129,18 +134,17 @@ void* work_get(size_t bytes, hipStream_t s) {
       continue;
     }
     const Block& c = d.kept[best];
-    const bool own = b.idle || b.stream == s, own_c = c.idle || c.stream == s;
-    if (own != own_c ? own : b.size < c.size) best = i;
+    if (b.idle != c.idle ? b.idle : b.size < c.size) best = i;
   }
   Block b;
   if (best >= 0) {
     b = d.kept[best];
+    if (!b.idle && hipStreamWaitEvent(s, b.ev, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      TOMHIP_CHECK(hipEventSynchronize(b.ev));
+    }
     d.kept.erase(d.kept.begin() + best);
     d.bytes -= b.size;
-    if (!b.idle && b.stream != s && hipStreamWaitEvent(s, b.ev, 0) != hipSuccess) {
-      (void)hipGetLastError();
-      (void)hipEventSynchronize(b.ev);
-    }
   } else {
     hipError_t e = hipMalloc(&b.p, want);
     if (e != hipSuccess && !d.kept.empty()) {
