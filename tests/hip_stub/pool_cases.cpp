@@ -83,11 +83,29 @@ static int per_thread() {
   return 0;
 }
 
+// A plan's blocks are kept for the next call only where the device could be
+// waited for.
+static int all_of_a_plan() {
+  FakeStream s;
+  work_device_up(0);
+  void* p = work_get(4096, &s);
+  void* q = work_get(8192, &s);
+  ++s.queued;
+  work_put_all({p, nullptr, q});
+  HOLDS(fake().frees == 0 && work_get(4096, &s) == p && work_get(8192, &s) == q && fake().waits == 0);
+  fake().sync_fails = true;
+  work_put_all({p, nullptr, q});
+  HOLDS(fake().frees == 2 && fake().live.empty());
+  work_device_down(0);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*f)();
-  } cases[] = {{"renew", renew}, {"same_handle", same_handle}, {"per_thread", per_thread}};
+  } cases[] = {{"renew", renew}, {"same_handle", same_handle}, {"per_thread", per_thread},
+                 {"all_of_a_plan", all_of_a_plan}};
   for (auto& c : cases)
     if (argc == 2 && !strcmp(argv[1], c.name)) return c.f();
   printf("no such case\n");

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <initializer_list>
+
 namespace tomhip {
 
 // A device workspace of at least `bytes` on the current device, for work on
@@ -23,8 +25,10 @@ void work_renew(T** p, size_t bytes, hipStream_t s) {
   *p = nullptr;
   work_get(p, bytes, s);
 }
-// work_put for a workspace that nothing queued anywhere uses.
-void work_put_idle(const void* p) noexcept;
+// Gives workspaces of the current device back that any of its streams may
+// still use: waits for the device, and where that is refused (while a stream
+// is being captured) they go to the driver instead of the next call.
+void work_put_all(std::initializer_list<const void*> ps) noexcept;
 
 // Contexts of a device, counted: the last one to go frees what is kept.
 void work_device_up(int device);

@@ -76,7 +76,9 @@ void keep(int device, Block b) {
   d.kept.push_back(b);
 }
 
-void put(const void* p, hipStream_t s, bool idle) noexcept {
+// what may still use a block that is given back
+enum Use { U_NONE, U_STREAM, U_UNKNOWN };
+void put(const void* p, hipStream_t s, Use use) noexcept {
   if (!p) return;
   State& S = state();
   std::lock_guard<std::mutex> g(S.mu);
@@ -90,14 +92,14 @@ void put(const void* p, hipStream_t s, bool idle) noexcept {
   S.used.erase(it);
   // the per-thread handle names another stream in each thread: what this
   // thread's has done says nothing of the work another thread queued
-  if (!idle && s == hipStreamPerThread) {
+  if (use == U_UNKNOWN || (use == U_STREAM && s == hipStreamPerThread)) {
     drop(b);  // hipFree waits for the device
     return;
   }
   // a stream that has run dry needs no event: most calls wait for their results
   // before they give their workspaces back (with an event each, a refinement
   // of 7 candidates took 646 us for 605, 16 subtomograms of 32^3 540 for 415)
-  b.idle = idle || hipStreamQuery(s) == hipSuccess;
+  b.idle = use == U_NONE || hipStreamQuery(s) == hipSuccess;
   if (!b.idle) {
     (void)hipGetLastError();  // not ready
     if (!b.ev && hipEventCreateWithFlags(&b.ev, hipEventDisableTiming) != hipSuccess) b.ev = nullptr;
@@ -164,8 +166,12 @@ void* work_get(size_t bytes, hipStream_t s) {
   return b.p;
 }
 
-void work_put(const void* p, hipStream_t s) noexcept { put(p, s, false); }
-void work_put_idle(const void* p) noexcept { put(p, nullptr, true); }
+void work_put(const void* p, hipStream_t s) noexcept { put(p, s, U_STREAM); }
+void work_put_all(std::initializer_list<const void*> ps) noexcept {
+  const Use use = hipDeviceSynchronize() == hipSuccess ? U_NONE : U_UNKNOWN;
+  if (use == U_UNKNOWN) (void)hipGetLastError();
+  for (const void* p : ps) put(p, nullptr, use);
+}
 
 void work_device_up(int device) {
   State& S = state();

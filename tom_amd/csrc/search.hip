@@ -1060,43 +1060,20 @@ void Search::bind_stream(hipStream_t s) {
 Search::~Search() { release(); }
 
 void Search::release() {
-  // whatever stream the plan last ran on may be gone by now: all work is done
-  // before its buffers are given back
-  (void)hipDeviceSynchronize();
-  work_put_idle(FI_);
-  work_put_idle(FIn_);
-  work_put_idle(maxc_);
-  work_put_idle(argm_);
-  work_put_idle(tmpl_);
-  work_put_idle(tpairs_);
-  tpairs_ = nullptr;
-  work_put_idle(t1_);
-  work_put_idle(tbox_);
-  work_put_idle(Ty_);
-  work_put_idle(Tyn_);
-  work_put_idle(Tx_);
-  work_put_idle(Q_);
-  work_put_idle(Pn_);
-  work_put_idle(gmax_);
-  work_put_idle(garg_);
-  work_put_idle(mu_);
-  work_put_idle(sig_);
-  work_put_idle(wsh_);
-  work_put_idle(rm_);
-  work_put_idle(ref_tt_);
-  work_put_idle(ref_work_);
-  work_put_idle(const_cast<float*>(mask_));
+  // whatever stream the plan last ran on may be gone by now
+  work_put_all({FI_, FIn_, maxc_, argm_, tmpl_, tpairs_, t1_, tbox_, Ty_, Tyn_, Tx_, Q_, Pn_, gmax_, garg_, mu_, sig_,
+                wsh_, rm_, ref_tt_, ref_work_, mask_, desc_});
+  drop_graph();
   FI_ = FIn_ = nullptr;
   maxc_ = nullptr;
   argm_ = nullptr;
   tmpl_ = t1_ = wsh_ = rm_ = ref_tt_ = nullptr;
+  tpairs_ = nullptr;
   tbox_ = Ty_ = Tyn_ = Tx_ = Q_ = Pn_ = ref_work_ = nullptr;
   gmax_ = nullptr;
   garg_ = nullptr;
   mu_ = sig_ = nullptr;
   mask_ = nullptr;
-  drop_graph();
-  work_put_idle(desc_);
   desc_ = nullptr;
   for (auto& e : evpool_) {
     (void)hipEventDestroy(e.a);
