@@ -100,12 +100,36 @@ static int all_of_a_plan() {
   return 0;
 }
 
+// Memory that is no workspace (a network's, a table's) is found where the
+// workspaces that wait for a next call hold it.
+static int other_memory() {
+  FakeStream s;
+  work_device_up(0);
+  fake().limit = 8 << 20;
+  void* p = work_get(6 << 20, &s);
+  work_put(p, &s);
+  HOLDS(fake().used == 6 << 20);
+  void* q = device_malloc(4 << 20);
+  HOLDS(q && fake().used == 4 << 20);
+  bool threw = false;
+  try {
+    device_malloc(8 << 20);
+  } catch (const Error&) {
+    threw = true;
+  }
+  HOLDS(threw);
+  (void)hipFree(q);
+  work_device_down(0);
+  HOLDS(fake().live.empty() && fake().freed_twice.empty());
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*f)();
   } cases[] = {{"renew", renew}, {"same_handle", same_handle}, {"per_thread", per_thread},
-                 {"all_of_a_plan", all_of_a_plan}};
+                 {"all_of_a_plan", all_of_a_plan}, {"other_memory", other_memory}};
   for (auto& c : cases)
     if (argc == 2 && !strcmp(argv[1], c.name)) return c.f();
   printf("no such case\n");

@@ -17,7 +17,16 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("case", ["renew", "same_handle", "per_thread", "all_of_a_plan"])
+@pytest.mark.parametrize("case", ["renew", "same_handle", "per_thread", "all_of_a_plan", "other_memory"])
 def test_pool(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_all_device_memory_comes_through_the_pool():
+    """A hipMalloc elsewhere would fail while the pool holds what it needs."""
+    csrc = os.path.join(ROOT, "tom_amd", "csrc")
+    for f in sorted(os.listdir(csrc)):
+        if f != "pool.hip":
+            for line in open(os.path.join(csrc, f)):
+                assert "hipMalloc(" not in line.split("//")[0], (f, line)

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "fft.h"
+#include "pool.h"
 
 namespace tomhip {
 
@@ -166,8 +167,7 @@ class Twiddles {
  private:
   template <typename T>
   static cpx<T>* upload(const std::vector<cpx<T>>& h) {
-    cpx<T>* d = nullptr;
-    TOMHIP_CHECK(hipMalloc(&d, sizeof(cpx<T>) * h.size()));
+    cpx<T>* d = static_cast<cpx<T>*>(device_malloc(sizeof(cpx<T>) * h.size()));
     TOMHIP_CHECK(hipMemcpy(d, h.data(), sizeof(cpx<T>) * h.size(), hipMemcpyHostToDevice));
     return d;
   }

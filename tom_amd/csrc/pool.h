@@ -7,8 +7,13 @@
 
 namespace tomhip {
 
+// hipMalloc on the current device, for memory of any lifetime: where it fails
+// the workspaces that wait for a next call are freed and it is tried again
+// (throws like TOMHIP_CHECK(hipMalloc)). Freed with hipFree.
+void* device_malloc(size_t bytes);
+
 // A device workspace of at least `bytes` on the current device, for work on
-// stream s (throws like TOMHIP_CHECK(hipMalloc)).
+// stream s (throws like device_malloc).
 void* work_get(size_t bytes, hipStream_t s);
 template <typename T>
 void work_get(T** p, size_t bytes, hipStream_t s) {

@@ -8,7 +8,7 @@
 // waits for whatever stream it names (equal handles may be different streams),
 // so calls on several streams and threads may share the pool. At most kKeep
 // bytes wait per device, oldest out first; all of it goes when an allocation
-// fails or the device's last context is destroyed.
+// of this library fails or the device's last context is destroyed.
 #include <map>
 #include <mutex>
 #include <vector>
@@ -53,6 +53,18 @@ void drop_all(Device& d) {
   for (Block& b : d.kept) drop(b);
   d.kept.clear();
   d.bytes = 0;
+}
+
+void* malloc_or_drop(Device& d, size_t bytes) {
+  void* p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e != hipSuccess && !d.kept.empty()) {
+    (void)hipGetLastError();
+    drop_all(d);
+    e = hipMalloc(&p, bytes);
+  }
+  TOMHIP_CHECK(e);
+  return p;
 }
 
 size_t rounded(size_t n) {
@@ -118,6 +130,14 @@ void put(const void* p, hipStream_t s, Use use) noexcept {
 
 }  // namespace
 
+void* device_malloc(size_t bytes) {
+  State& S = state();
+  int device = 0;
+  TOMHIP_CHECK(hipGetDevice(&device));
+  std::lock_guard<std::mutex> g(S.mu);
+  return malloc_or_drop(S.dev[device], bytes);
+}
+
 void* work_get(size_t bytes, hipStream_t s) {
   State& S = state();
   const size_t want = rounded(bytes ? bytes : 1);
@@ -148,13 +168,7 @@ void* work_get(size_t bytes, hipStream_t s) {
     d.kept.erase(d.kept.begin() + best);
     d.bytes -= b.size;
   } else {
-    hipError_t e = hipMalloc(&b.p, want);
-    if (e != hipSuccess && !d.kept.empty()) {
-      (void)hipGetLastError();
-      drop_all(d);
-      e = hipMalloc(&b.p, want);
-    }
-    TOMHIP_CHECK(e);
+    b.p = malloc_or_drop(d, want);
     b.size = want;
   }
   try {

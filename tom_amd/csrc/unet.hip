@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "common.h"
+#include "pool.h"
 #include "unet.h"
 
 namespace tomhip {
@@ -1471,8 +1472,7 @@ struct Unet::Impl {
 
   template <typename T>
   T* alloc(size_t n) {
-    void* p = nullptr;
-    TOMHIP_CHECK(hipMalloc(&p, n * sizeof(T) + 16));
+    void* p = device_malloc(n * sizeof(T) + 16);
     owned.push_back(p);
     return static_cast<T*>(p);
   }
