@@ -31,13 +31,20 @@ typedef struct tomhip_search tomhip_search;
 
 /* ---------------------------------------------------------------- context */
 /* One context per device and stream. No reference counterpart (the MEX
- * gateways are stateless); the context owns twiddle tables and workspaces. */
+ * gateways are stateless); the context owns twiddle tables. Workspaces of the
+ * calls are kept between calls, up to 4 GiB per device for all its contexts
+ * together: they are freed when an allocation of this library fails, by
+ * tomhip_release_workspaces and with the device's last context. Other
+ * allocators of the process cannot reach them by themselves. */
 int tomhip_init(int device, tomhip_ctx** ctx);
 void tomhip_destroy(tomhip_ctx* ctx);
 const char* tomhip_last_error(tomhip_ctx* ctx);
 /* Launch on a caller-owned hipStream_t (NULL = the context's own stream). */
 int tomhip_set_stream(tomhip_ctx* ctx, void* hip_stream);
 int tomhip_synchronize(tomhip_ctx* ctx);
+/* Frees the workspaces kept on the context's device (those in use by a call or
+ * a search plan stay); waits for the device. */
+int tomhip_release_workspaces(tomhip_ctx* ctx);
 
 /* ---------------------------------------------------------------- rotation */
 /* tom_rotatec(in, out, euler, 'linear', center): replaces the MEX core of

@@ -124,12 +124,27 @@ static int other_memory() {
   return 0;
 }
 
+// What waits can be asked for; what is in use stays.
+static int trim() {
+  FakeStream s;
+  work_device_up(0);
+  void* p = work_get(4096, &s);
+  work_put(work_get(8192, &s), &s);
+  HOLDS(fake().live.size() == 2);
+  work_trim(0);
+  HOLDS(fake().live.size() == 1 && fake().live.count(p));
+  work_put(p, &s);
+  HOLDS(work_get(4096, &s) == p);
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*f)();
   } cases[] = {{"renew", renew}, {"same_handle", same_handle}, {"per_thread", per_thread},
-                 {"all_of_a_plan", all_of_a_plan}, {"other_memory", other_memory}};
+                 {"all_of_a_plan", all_of_a_plan}, {"other_memory", other_memory},
+                 {"trim", trim}};
   for (auto& c : cases)
     if (argc == 2 && !strcmp(argv[1], c.name)) return c.f();
   printf("no such case\n");

@@ -17,7 +17,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("case", ["renew", "same_handle", "per_thread", "all_of_a_plan", "other_memory"])
+@pytest.mark.parametrize("case", ["renew", "same_handle", "per_thread", "all_of_a_plan", "other_memory", "trim"])
 def test_pool(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

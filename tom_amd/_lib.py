@@ -24,6 +24,7 @@ SIGNATURES = {
     "tomhip_last_error": (ctypes.c_char_p, [vp]),
     "tomhip_set_stream": (ctypes.c_int, [vp, vp]),
     "tomhip_synchronize": (ctypes.c_int, [vp]),
+    "tomhip_release_workspaces": (ctypes.c_int, [vp]),
     "tomhip_rotate3d_f32": (ctypes.c_int, [vp, vp, vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, vp,
                                            ctypes.c_int, vp]),
     "tomhip_rotate2d_f32": (ctypes.c_int, [vp, vp, vp, ctypes.c_int64, ctypes.c_int64, vp, ctypes.c_int, vp]),

@@ -57,6 +57,11 @@ class Context:
             s = torch.cuda.current_stream(self.device).cuda_stream
             self.check(self.lib.tomhip_set_stream(self.h, ctypes.c_void_p(s)))
 
+    def release_workspaces(self):
+        """Frees the device memory that calls keep for the next one (up to
+        4 GiB per device), for other allocators such as torch's."""
+        self.check(self.lib.tomhip_release_workspaces(self.h))
+
     def close(self):
         if self.h:
             self.lib.tomhip_destroy(self.h)

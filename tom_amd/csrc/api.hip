@@ -175,6 +175,13 @@ int tomhip_synchronize(tomhip_ctx* ctx) {
   });
 }
 
+int tomhip_release_workspaces(tomhip_ctx* ctx) {
+  return guard(ctx, [&] {
+    TOMHIP_REQUIRE(ctx, ERR_WRONG_INPUT, "null context");
+    work_trim(ctx->device);
+  });
+}
+
 int tomhip_rotate3d_f32(tomhip_ctx* ctx, const float* src, float* dst, int64_t nx, int64_t ny, int64_t nz,
                         const float* euler, int neuler, const float* center) {
   return guard(ctx, [&] {

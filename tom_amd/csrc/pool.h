@@ -35,6 +35,9 @@ void work_renew(T** p, size_t bytes, hipStream_t s) {
 // is being captured) they go to the driver instead of the next call.
 void work_put_all(std::initializer_list<const void*> ps) noexcept;
 
+// Frees what waits for a next call on the device.
+void work_trim(int device);
+
 // Contexts of a device, counted: the last one to go frees what is kept.
 void work_device_up(int device);
 void work_device_down(int device) noexcept;

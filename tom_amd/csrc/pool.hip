@@ -8,7 +8,8 @@
 // waits for whatever stream it names (equal handles may be different streams),
 // so calls on several streams and threads may share the pool. At most kKeep
 // bytes wait per device, oldest out first; all of it goes when an allocation
-// of this library fails or the device's last context is destroyed.
+// of this library fails, when tomhip_release_workspaces asks for it or when the
+// device's last context is destroyed.
 #include <map>
 #include <mutex>
 #include <vector>
@@ -185,6 +186,12 @@ void work_put_all(std::initializer_list<const void*> ps) noexcept {
   const Use use = hipDeviceSynchronize() == hipSuccess ? U_NONE : U_UNKNOWN;
   if (use == U_UNKNOWN) (void)hipGetLastError();
   for (const void* p : ps) put(p, nullptr, use);
+}
+
+void work_trim(int device) {
+  State& S = state();
+  std::lock_guard<std::mutex> g(S.mu);
+  drop_all(S.dev[device]);
 }
 
 void work_device_up(int device) {
