@@ -12,6 +12,7 @@
 // optional mask multiplies the result (t = rot(T) .* M of the
 // template-matching loop).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "rotate.h"
@@ -43,8 +44,9 @@ __global__ void k_pairs_x(const float* src, int sx, long n, float2* pairs) {
     pairs[b] = make_float2(src[b], (b % sx) == sx - 1 ? 0.f : src[b + 1]);
 }
 
-// A block takes 16 x 16 voxels of rz planes of one rotation, a thread the rz
-// voxels of its column: of a source coordinate, px + rm00 i + rm10 j + rm20 k
+// A thread takes rz planes of one column of one rotation, a block 16 x 16
+// columns (grid: tiles, plane groups, rotations) or, with FLAT, 256 of the
+// columns of all plane groups numbered through (grid.x): of a source coordinate, px + rm00 i + rm10 j + rm20 k
 // summed in this order, only the last sum changes with the plane, and the
 // gathers of RU planes (4, or rz = 1) are in flight together. They are unconditional: a tap
 // past the last row or plane is read at the row or plane itself and then
@@ -54,14 +56,24 @@ __global__ void k_pairs_x(const float* src, int sx, long n, float2* pairs) {
 // index divisions, branches per axis) and this: 1.03 and 0.80 ms, bound by the
 // gathers. Single 4-byte-aligned loads of the source in place of the pairs,
 // and 8 x 8 patches: 0.78 and 0.84 ms.
-template <bool PAIRS, int RU>
+template <bool PAIRS, int RU, bool FLAT>
 __global__ __launch_bounds__(NT_ROT) void k_rotate_direct(RotParams P, int rz_) {
   const int sx = P.sx, sy = P.sy, sz = P.sz, sxy = sx * sy;
   const float px = P.px, py = P.py, pz = P.pz;
-  const int nbx = (sx + 15) / 16;
-  const int i = blockIdx.x % nbx * 16 + threadIdx.x % 16, j = blockIdx.x / nbx * 16 + threadIdx.x / 16;
-  const int k0 = blockIdx.y * rz_;
-  if (i >= sx || j >= sy) return;
+  int i, j, k0;
+  if constexpr (FLAT) {
+    const unsigned q = blockIdx.x * NT_ROT + threadIdx.x, c = q % (unsigned)sxy;
+    i = c % (unsigned)sx;
+    j = c / (unsigned)sx;
+    k0 = (int)(q / (unsigned)sxy) * rz_;
+    if (k0 >= sz) return;
+  } else {
+    const int nbx = (sx + 15) / 16;
+    i = blockIdx.x % nbx * 16 + threadIdx.x % 16;
+    j = blockIdx.x / nbx * 16 + threadIdx.x / 16;
+    k0 = blockIdx.y * rz_;
+    if (i >= sx || j >= sy) return;
+  }
   const float* img = P.src;
   const float2* pr = P.pairs;
   const float pi = (float)(int)((float)i - px);
@@ -271,16 +283,39 @@ void launch_rotate(const float* src, float* dst, const float* rm_dev, int nrot, 
   P.rm_step = rm_step;
   P.nrot = nrot;
   P.pairs = pairs;
+  // Tiles of 16 x 16 columns where the tiles are full, and for volumes that an
+  // XCD's L2 does not hold (there the patch matters more than idle lanes);
+  // otherwise the columns numbered through, so that no lane is idle. 6 million
+  // voxels with pairs, in us, a voxel per thread / tiles / numbered: 17^3 36 /
+  // 74 / 34, 24^3 36 / 44 / 28, 40^3 35 / 33 / 33, 44^3 34 / 31 / 33, 48^3 34 /
+  // 31 / 34, 50^3 36 / 50 / 35, 60^3 32 / 35 / 31, 64^3 34 / 30 / 33; 10 million
+  // without: 100^3 241 / 200 / 198, 112^3 379 / 264 / 284.
+  const long sxy = (long)sx * sy, plane = (long)((sx + 15) / 16) * ((sy + 15) / 16);
+  const double full = sxy / (256.0 * plane);
+  const bool flat = full < 0.95 && (full < 0.5 || sxy * sz <= (1L << 20)) && sxy * sz < (1L << 31);
+  auto blocks = [&](int rz) {
+    const long groups = (sz + rz - 1) / rz;
+    return flat ? (sxy * groups + NT_ROT - 1) / NT_ROT : plane * groups;
+  };
   // 8 planes a thread, one where the blocks are few (batches of 16, 4 planes
-  // and one, in us: 24^3 7.7 and 6.9, 16^3 7.1 and 6.1)
-  const long plane = (long)((sx + 15) / 16) * ((sy + 15) / 16);
-  const int rz = plane * ((sz + 7) / 8) * nrot >= 2048 ? 8 : 1;
-  dim3 grid((unsigned)plane, (unsigned)((sz + rz - 1) / rz), (unsigned)std::min(nrot, 65535));
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(NT_ROT), 0, stream, P, rz); };
-  if (pairs)
-    rz > 1 ? go(k_rotate_direct<true, 4>) : go(k_rotate_direct<true, 1>);
-  else
-    rz > 1 ? go(k_rotate_direct<false, 4>) : go(k_rotate_direct<false, 1>);
+  // and one, in us: 24^3 7.7 and 6.9, 16^3 7.1 and 6.1), the planes, or, of
+  // numbered columns, the share of threads that have a whole column (12^3 41
+  // and 33, 17^3 41 and 34, 20^3 30 and 34) or where a wave's columns leave
+  // its plane's neighbourhood (60^3 36 and 31)
+  int rz = sz >= 3 && blocks(8) * nrot >= 2048 ? 8 : 1;
+  if (flat && (sxy * sz < 0.75 * 8 * NT_ROT * blocks(8) || (sxy > 1400 && sz > 8))) rz = 1;
+  while (!flat && (sz + rz - 1) / rz > 65535) rz *= 2;
+  const dim3 grid((unsigned)(flat ? blocks(rz) : plane), flat ? 1u : (unsigned)((sz + rz - 1) / rz),
+                  (unsigned)std::min(nrot, 65535));
+  auto go = [&](auto pairs_c, auto ru, auto flat_c) {
+    hipLaunchKernelGGL((k_rotate_direct<decltype(pairs_c)::value, decltype(ru)::value, decltype(flat_c)::value>), grid,
+                       dim3(NT_ROT), 0, stream, P, rz);
+  };
+  auto with = [&](auto pairs_c, auto flat_c) {
+    rz > 1 ? go(pairs_c, std::integral_constant<int, 4>{}, flat_c) : go(pairs_c, std::integral_constant<int, 1>{}, flat_c);
+  };
+  auto on = [&](auto pairs_c) { flat ? with(pairs_c, std::true_type{}) : with(pairs_c, std::false_type{}); };
+  pairs ? on(std::true_type{}) : on(std::false_type{});
   TOMHIP_CHECK(hipGetLastError());
 }
 
