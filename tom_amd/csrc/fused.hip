@@ -426,7 +426,9 @@ template <int XH, int Y>
 __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __restrict__ Q, float* __restrict__ maxc,
                                                                 int32_t* __restrict__ argm,
                                                                 const c32* tw, int Z, int ka, int first_index,
-                                                                const long* desc) {
+                                                                const long* desc, int apb, float* __restrict__ pv,
+                                                                uint8_t* __restrict__ pi, long n) {
+  const int a0 = blockIdx.y * apb, a1 = min(a0 + apb, ka);
   if (desc) first_index = (int)(desc[1] + desc[0] * ka);
   using I1 = ClassStage<XH, Y, 1>;
   constexpr int NW = waves_bc(XH), NT_ = 64 * NW, R0 = I1::R0, Lp = I1::Lp, ZB = I1::ZB;
@@ -468,7 +470,7 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
     }
     return ((I1::NQ * NCH1) % NW == 0 || k < I1::NQ * NCH1) && zl < (PAIR ? nzb / 2 : nzb);
   };
-  const c32* qp = Q + (long)z0 * 2 * SU + (long)rc * Lp * XH * 2 + bit;
+  const c32* qp = Q + a0 * Z * SU + (long)z0 * 2 * SU + (long)rc * Lp * XH * 2 + bit;
   // quarter part of the loads of one angle (all of them: part < 0)
   auto fetch = [&](const c32* qa, int part, int w, int lane) {
 #pragma unroll
@@ -489,7 +491,7 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
   };
   // the next angle's loads are issued a quarter at a time between the stages
   auto ahead = [&](int a, int part, int w, int lane) {
-    if (a + 1 < ka) fetch(qp, part, fresh_uniform(w), fresh(lane));
+    if (a + 1 < a1) fetch(qp, part, fresh_uniform(w), fresh(lane));
   };
   float bx[EPT], by[EPT];
   constexpr int NI = (EPT + 7) / 8;
@@ -497,11 +499,11 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
 #pragma unroll
   for (int p = 0; p < NI; ++p) ix[p] = iy[p] = 0u;
 #pragma unroll
-  for (int k = 0; k < EPT; ++k) bx[k] = by[k] = 0.f;
+  for (int k = 0; k < EPT; ++k) bx[k] = by[k] = -INFINITY;
   fetch(qp, -1, w_, lane_);
-  for (int a = 0; a < ka; ++a) {
+  for (int a = a0; a < a1; ++a) {
     const int lane = fresh(lane_), w = fresh_uniform(w_);
-    if (a) __syncthreads();  // the previous angle's lines have been read
+    if (a > a0) __syncthreads();  // the previous angle's lines have been read
 #pragma unroll
     for (int t = 0; t < M1; ++t) {
       int q, zl, col;
@@ -605,7 +607,9 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
         });
     ahead(a, 3, w, lane);
   }
-  // the batch's maximum against the resident maps, a quarter of every line at
+  const int first = pv ? 0 : first_index;
+  // the batch's maximum against the resident maps (a group's, for
+  // merge_groups, to pv and pi), a quarter of every line at
   // a time through LDS so that the maps are read and written in rows
   constexpr int KC = EPT / 4, NS = NW * KC, FP = NS + 1;
   static_assert(EPT % 4 == 0 && 64 * FP * 2 <= 64 * P, "staging area");
@@ -618,17 +622,22 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
     for (int i = 0; i < KC; ++i) {
       const int k = r * KC + i, e = lane_ * FP + w_ + NW * i;
       sval[e] = make_float2(bx[k], by[k]);
-      sidx[e] = make_int2(first_index + (int)((ix[k / 8] >> (4 * (k % 8))) & 15u),
-                          first_index + (int)((iy[k / 8] >> (4 * (k % 8))) & 15u));
+      sidx[e] = make_int2(first + (int)((ix[k / 8] >> (4 * (k % 8))) & 15u),
+                          first + (int)((iy[k / 8] >> (4 * (k % 8))) & 15u));
     }
     __syncthreads();
     for (int i = threadIdx.x; i < nzb * Lp * NS; i += NT_) {
       const int l = i / NS, e = i % NS;
       const long line = (long)plane(l / Lp) * Y + (l % Lp) * R0 + rc;
       const long vx = (line * XH + r * NS + e) * 2;
-      const float2 cur = *reinterpret_cast<const float2*>(maxc + vx);
       const float2 nv = sval[l * FP + e];
       const int2 ni = sidx[l * FP + e];
+      if (pv) {
+        *reinterpret_cast<float2*>(pv + blockIdx.y * n + vx) = nv;
+        *reinterpret_cast<uchar2*>(pi + blockIdx.y * n + vx) = make_uchar2(ni.x, ni.y);
+        continue;
+      }
+      const float2 cur = *reinterpret_cast<const float2*>(maxc + vx);
       if (nv.x > cur.x) {
         maxc[vx] = nv.x;
         argm[vx] = ni.x;
@@ -641,11 +650,12 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
   }
 }
 
-// The lengths that have the fused kernels. Z: 16 elements a lane (24 at 192);
-// the others of the search's lengths leave waves or lanes idle and measured
-// slower than the separate passes (batches of 16, fused / separate in us:
-// 512x192x48 560 / 445, 320x320x80 772 / 697, 256x96x96 292 / 236). Y: first
-// radix 8 or 4, at most 64 rows in a class, the next radix 8 or 4.
+// The lengths that have the fused kernels. Z: 16 elements a lane (24 at 192).
+// 48, 80 and 96 leave waves or lanes idle and measured slower than the separate
+// passes (batches of 16, fused / separate in us: 512x192x48 560 / 445,
+// 320x320x80 772 / 697, 256x96x96 292 / 236); 120, 160, 200 and 240 fit LDS and
+// have not been measured. Y: first radix 8 or 4, at most 64 rows in a class,
+// the next radix 8 or 4.
 #define TOMHIP_CASE(n)                   \
   case n:                                \
     f(std::integral_constant<int, n>{}); \
@@ -712,24 +722,59 @@ void fused_prepare(Twiddles& tw, int X, int Y, int Z) {
   (void)bc_list(tw, X, Y);
 }
 
+// Angles per block of k_fused_a. Few blocks: the batch's angles over more of
+// them, to twice what the CUs hold at once by their LDS at Z = 32 and 64
+// (batches of 16, us, to 1,024 blocks and to this: 512x192x32 187 and 98,
+// 512x160x64 214 and 127), 1,024 from 128 on (more read F_I more often:
+// 512x96x128 ka 8 83 and, to 2,048, 95).
+static int a_angles(int X, int Y, int Z, int ka) {
+  const int R0 = plan_radix(Y, 0), blocks = X / 2 / (64 / R0) * (Y / R0);
+  const int groups = std::min(ka, std::max(1, std::max(1024, 131072 / Z) / blocks));
+  return (ka + groups - 1) / groups;
+}
+// Blocks of k_fused_bc for one group of angles, and how many the CUs hold at
+// once by their LDS.
+static int bc_blocks(int Y, int Z) {
+  const int ZB = z_group(Y), half = z_paired(Y) ? ZB / 2 : ZB, sides = z_paired(Y) ? 1 : 2;
+  return (Z / 2 + half - 1) / half * sides * plan_radix(Y, 0);
+}
+static int bc_places(int X) { return 256 * (160 * 1024 / (64 * (X / 2 + 1) * (int)sizeof(c32))); }
+
+int fused_bc_groups(int X, int Y, int Z, int ka) {
+  // half a chip of blocks or less: two groups, merged by one more launch.
+  // Batches of 16, us, one group and two with the merge: 512x192x32 173 and
+  // 103, 128x240x128 216 and 128, 256x256x64 161 and 115; where the blocks
+  // fill more: 512x192x64 177 and 205. Three and four groups take longer.
+  return ka >= 4 && 2 * bc_blocks(Y, Z) <= bc_places(X) ? 2 : 1;
+}
+
 bool fused_supported(int X, int Y, int Z, int ka) {
   // The saved traffic pays once a batch's Q does not fit in the memory-side
   // cache (256 MB); below, the separate passes have more blocks to fill the
   // chip with. Batches, fused / separate in us: 134 MB 128x128x128 216 / 207,
-  // 512x64x64 242 / 235; 268 MB 256x128x128 337 / 344, 128x256x128 ka 16
-  // 325 / 317; 403 MB 256x256x192 ka 8 469 / 489; 537 MB 256x256x128
-  // 500 / 661; 4.3 GB 512x512x256 3218 / 4500.
+  // 512x64x64 242 / 235; 4.3 GB 512x512x256 3218 / 4500.
   if (8L * ka * Z * Y * (X / 2) < (192L << 20)) return false;
-  return dispatch_z(Z, [](auto) {}) && dispatch_x(X / 2, [](auto) {}) && dispatch_y(Y, [](auto) {});
+  if (!(dispatch_z(Z, [](auto) {}) && dispatch_x(X / 2, [](auto) {}) && dispatch_y(Y, [](auto) {}))) return false;
+  // 1,402 batches of all these lengths, 192 MB to 3 GB, whole runs, separate
+  // passes over fused kernels: Z = 32 and 64 1.03 to 1.46; from 128 on 0.80 to
+  // 1.54, slower with the fused ones at Z = 192 (one block of 8 waves a CU),
+  // with few angles to a block of fused_a, and with the last round of
+  // fused_bc's blocks nearly empty. The sum below is a fit to the difference,
+  // in ns per 10^6 bytes of Q (the separate passes take 1,000 to 1,400), and
+  // where it is positive the ratio is 0.93 to 1.54, below 0.98 in 31 of 910;
+  // where it is not, 0.80 to 1.15 in 255.
+  if (Z < 128) return true;
+  const int nb = bc_blocks(Y, Z) * fused_bc_groups(X, Y, Z, ka);
+  const int y = (Y & (Y - 1)) == 0 ? 250 : Y < 200 ? 320 : 390;  // fused_bc's own time
+  int gain = Z == 128 ? 480 : Z == 192 ? 390 : 580 - 500 / ka;
+  if ((X & (X - 1)) == 0 && X > 128) gain += 50;
+  return gain > y * ((nb + 255) / 256 * 256) / nb + 250 / a_angles(X, Y, Z, ka);
 }
 
 void fused_a(Twiddles& tw, hipStream_t s, const c32* Ty, const c32* Tyn, c32* Pn, const c32* FI, const c32* FIn,
              c32* Q, int X, int Y, int Z, int nz, int ka) {
   const int Xh = X / 2, R0 = plan_radix(Y, 0), T = 64 / R0;
-  const int blocks = Xh / T * (Y / R0);
-  // few blocks: spread the batch's angles over more of them
-  const int groups = std::min(ka, std::max(1, 1024 / blocks));
-  const int apb = (ka + groups - 1) / groups;
+  const int blocks = Xh / T * (Y / R0), apb = a_angles(X, Y, Z, ka);
   dispatch_z(Z, [&](auto Zc) {
     constexpr int L = decltype(Zc)::value;
     const dim3 bt(64 * waves_a(L));
@@ -744,15 +789,13 @@ void fused_a(Twiddles& tw, hipStream_t s, const c32* Ty, const c32* Tyn, c32* Pn
 }
 
 void fused_bc(Twiddles& tw, hipStream_t s, const c32* Q, float* maxc, int32_t* argm, int X, int Y, int Z, int ka,
-              int first_index, const long* desc) {
+              int first_index, const long* desc, int apb, float* pv, uint8_t* pi) {
   dispatch_x(X / 2, [&](auto Xc) {
     dispatch_y(Y, [&](auto Yc) {
-      constexpr int XH = decltype(Xc)::value, YL = decltype(Yc)::value, ZB = z_group(YL);
-      const int half = z_paired(YL) ? ZB / 2 : ZB, sides = z_paired(YL) ? 1 : 2;
-      hipLaunchKernelGGL((k_fused_bc<XH, YL>),
-                         dim3((unsigned)((Z / 2 + half - 1) / half * sides * plan_radix(YL, 0))),
+      constexpr int XH = decltype(Xc)::value, YL = decltype(Yc)::value;
+      hipLaunchKernelGGL((k_fused_bc<XH, YL>), dim3((unsigned)bc_blocks(YL, Z), (unsigned)((ka + apb - 1) / apb)),
                          dim3(64 * waves_bc(XH)), 0, s, Q, maxc, argm, bc_list(tw, X, YL), Z, ka, first_index,
-                         desc);
+                         desc, apb, pv, pi, (long)X * Y * Z);
     });
   });
   TOMHIP_CHECK(hipGetLastError());

@@ -46,12 +46,13 @@ __global__ void k_pairs_x(const float* src, int sx, long n, float2* pairs) {
 
 // A thread takes rz planes of one column of one rotation, a block 16 x 16
 // columns (grid: tiles, plane groups, rotations) or, with FLAT, 256 of the
-// columns of all plane groups numbered through (grid.x): of a source coordinate, px + rm00 i + rm10 j + rm20 k
-// summed in this order, only the last sum changes with the plane, and the
-// gathers of RU planes (4, or rz = 1) are in flight together. They are unconditional: a tap
-// past the last row or plane is read at the row or plane itself and then
-// replaced by 0, and a voxel outside reads element 0. A wave's 16 x 4 patch
-// keeps its gathers near each other whichever way the volume is turned.
+// columns of all plane groups numbered through (grid.x): of a source
+// coordinate, px + rm00 i + rm10 j + rm20 k summed in this order, only the last
+// sum changes with the plane, and the gathers of RU planes (4, or rz = 1) are
+// in flight together. They are unconditional: a tap past the last row or plane
+// is read at the row or plane itself and then replaced by 0, and a voxel
+// outside reads element 0. A tile's wave, a patch of 16 x 4, keeps its gathers
+// near each other whichever way the volume is turned.
 // 1,728 rotations of 48^3 with pairs and mask, with a voxel per thread (64-bit
 // index divisions, branches per axis) and this: 1.03 and 0.80 ms, bound by the
 // gathers. Single 4-byte-aligned loads of the source in place of the pairs,

@@ -102,6 +102,7 @@ class Search {
   void launch_passB(int ka, int z0, int zn);
   void launch_passC(int ka, int z0, int zn, long first_index, const long* desc);
   int passC_groups(int ka) const;
+  void merge_groups(int groups, int ka, long v0, long cnt, int first_index, const long* desc);
   void capture_graph();
   void drop_graph();
   template <class F>
@@ -144,7 +145,7 @@ class Search {
   c32* Tyn_ = nullptr;       // [KA][nz][Y]
   c32* Tx_ = nullptr;        // [KA][nz][ny][pitch] template x-DFT rows, when they do not fit in Q
   c32* Q_ = nullptr;         // [KA][Z][Y][Xh]
-  float* gmax_ = nullptr;    // [groups][N] maxima of pass C's angle groups
+  float* gmax_ = nullptr;    // [groups][N] maxima of a batch's angle groups
   uint8_t* garg_ = nullptr;  // [groups][N] and their places in the batch
   c32* Pn_ = nullptr;        // [KA][Z][Y] product at kx = X/2 (fused passes)
   bool started_ = false;

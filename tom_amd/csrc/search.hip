@@ -1020,8 +1020,12 @@ Search::Search(Twiddles& tw, hipStream_t s, const float* volume, int X_, int Y_,
     work_get(&Ty_, sizeof(c32) * (long)KA_ * nz * Y * Xh, s_);
     work_get(&Tyn_, sizeof(c32) * (long)KA_ * nz * Y, s_);
     work_get(&Q_, sizeof(c32) * (long)KA_ * Z * Y * Xh, s_);
-    if (fused_supported(X, Y, Z, KA_)) work_get(&Pn_, sizeof(c32) * (long)KA_ * Z * Y, s_);
-    if (const long g = passC_groups(KA_); g > 1) {
+    long g = passC_groups(KA_);
+    if (fused_supported(X, Y, Z, KA_)) {
+      work_get(&Pn_, sizeof(c32) * (long)KA_ * Z * Y, s_);
+      g = std::max(g, (long)fused_bc_groups(X, Y, Z, KA_));
+    }
+    if (g > 1) {
       work_get(&gmax_, sizeof(float) * g * N, s_);
       work_get(&garg_, g * N, s_);
     }
@@ -1398,8 +1402,9 @@ void Search::launch_passB(int ka, int z0, int zn) {
 
 bool Search::use_fused(int ka) const {
   // The fused kernels take the z transform of 256 as 16 x 16, which is what
-  // 16-wide tiles mean there; a z-chunk asks for the separate passes.
-  return zchunk_ == 0 && (Z != 256 || tile_a_ == 16) && fused_supported(X, Y, Z, ka);
+  // 16-wide tiles mean there; a z-chunk asks for the separate passes. A last
+  // batch may be one that gains where the full ones do not: it has no Pn_.
+  return Pn_ && zchunk_ == 0 && (Z != 256 || tile_a_ == 16) && fused_supported(X, Y, Z, ka);
 }
 
 void Search::run_batch(const float* rm_dev, int ka, long first_index, const long* desc) {
@@ -1454,7 +1459,12 @@ void Search::run_batch(const float* rm_dev, int ka, long first_index, const long
   });
   if (fused) {
     timed(K_PASSA, [&] { fused_a(tw_, s_, Ty_, Tyn_, Pn_, FI_, FIn_, Q_, X, Y, Z, nz, ka); });
-    timed(K_PASSC, [&] { fused_bc(tw_, s_, Q_, maxc_, argm_, X, Y, Z, ka, (int)first_index, desc); });
+    timed(K_PASSC, [&] {
+      const int groups = fused_bc_groups(X, Y, Z, ka), apb = (ka + groups - 1) / groups, ng = (ka + apb - 1) / apb;
+      fused_bc(tw_, s_, Q_, maxc_, argm_, X, Y, Z, ka, (int)first_index, desc, apb, ng > 1 ? gmax_ : nullptr,
+               ng > 1 ? garg_ : nullptr);
+      if (ng > 1) merge_groups(ng, ka, 0, N, (int)first_index, desc);
+    });
     return;
   }
   timed(K_PASSA, [&] { launch_passA(ka); });
@@ -1483,6 +1493,12 @@ int Search::passC_groups(int ka) const {
   return groups;
 }
 
+void Search::merge_groups(int groups, int ka, long v0, long cnt, int first_index, const long* desc) {
+  hipLaunchKernelGGL(k_merge_groups, dim3((unsigned)((cnt / 2 + NT - 1) / NT)), dim3(NT), 0, s_, (const float*)gmax_,
+                     (const uint8_t*)garg_, groups, N, v0, cnt, first_index, desc, ka, maxc_, argm_);
+  TOMHIP_CHECK(hipGetLastError());
+}
+
 void Search::launch_passC(int ka, int z0, int zn, long first_index, const long* desc) {
   dispatch_xh(Xh, [&](auto Lc) {
     constexpr int L = decltype(Lc)::value;
@@ -1500,10 +1516,7 @@ void Search::launch_passC(int ka, int z0, int zn, long first_index, const long* 
       go(k_passC<L, false>);
     } else {
       go(k_passC<L, true>);
-      const long cnt = nl * X;
-      hipLaunchKernelGGL(k_merge_groups, dim3((unsigned)((cnt / 2 + NT - 1) / NT)), dim3(NT), 0, s_,
-                         (const float*)gmax_, (const uint8_t*)garg_, ng, N, line0 * X, cnt, (int)first_index, desc, ka,
-                         maxc_, argm_);
+      merge_groups(ng, ka, line0 * X, nl * X, (int)first_index, desc);
     }
   });
   TOMHIP_CHECK(hipGetLastError());
