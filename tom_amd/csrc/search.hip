@@ -1351,6 +1351,34 @@ void Search::set_tiles(int ta, int tb) {
   tile_b_ = tb;
 }
 
+// Groups of a batch's angles for a kernel of `blocks` blocks a group, of which
+// a CU holds per_cu: those of the least time, where n blocks on a CU at once
+// take (n + 1) / 2 of the time of one, and a block's start (F_I, the first
+// planes) that of 0.7 angles. Pass A undivided and divided, in us: 64x64x64
+// ka 16 65 and 22, 64x320x128 ka 8 60 and 50, 512x32x16 ka 16 42 and 20; kept
+// whole: 160x240x160 ka 8 101 (by three groups 108), 96x200x192 ka 2 31 (33).
+static int angle_groups(int blocks, int ka, int per_cu) {
+  int best = 1;
+  double least = 0;
+  for (int g = 1; g <= ka; ++g) {
+    const int apb = (ka + g - 1) / g;
+    if ((ka + apb - 1) / apb != g) continue;
+    const int n = (blocks * g + 255) / 256, rem = n % per_cu;
+    const double t = (n / per_cu * (per_cu + 1) + (rem ? rem + 1 : 0)) * (apb + 0.7);
+    if (g == 1 || t < 0.97 * least) {
+      best = g;
+      least = t;
+    }
+  }
+  return best;
+}
+template <class K>
+static int blocks_per_cu(K kern) {
+  int n = 0;
+  TOMHIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, NT_A, 0));
+  return std::max(1, n);
+}
+
 void Search::launch_passA(int ka) {
   dispatch_tile(tile_a_, [&](auto TWc) {
     constexpr int TW = decltype(TWc)::value;
@@ -1363,20 +1391,18 @@ void Search::launch_passA(int ka) {
           hipLaunchKernelGGL(k_passA4<false>, dim3(Xh / TW - 1, Y), dim3(256), 0, s_, (const c32*)Ty_,
                              (const c32*)Tyn_, (const c32*)FI_, (const c32*)FIn_, Q_, tw_.f32(L), Y, Xh, nz, ka);
       } else if constexpr ((long)L * (TW + 1) * 8 + (long)L * 8 <= kLdsMax) {
-        // few blocks: spread the batch's angles over as many as the CUs hold
-        // at once. Batches of 16, undivided and divided, in us: 64x64x64 68
-        // and 29, 128x128x64 68 and 50. One launch for both kinds of tile
-        // takes 20 at 64x64x64 but 67 for 61 at 320x240x96 ka 4.
-        constexpr long lds = (passA_fi_lds<L, TW>() ? 2 : 1) * (long)L * (TW + 1) * 8 + L * 8;
-        constexpr int per_cu = (int)std::min(2048L / NT_A, 160 * 1024 / lds);
-        auto go = [&](auto kern, int tiles) {
-          const int groups = std::min(ka, std::max(1, 256 * per_cu / (tiles * Y)));
+        // One launch for both kinds of tile takes 20 us at 64x64x64 but 67 for
+        // 61 at 320x240x96 ka 4.
+        auto go = [&](auto nyq, int tiles) {
+          auto* kern = k_passA<L, TW, decltype(nyq)::value>;
+          static const int per_cu = blocks_per_cu(kern);
+          const int groups = angle_groups(tiles * Y, ka, per_cu);
           const int apb = (ka + groups - 1) / groups;
           hipLaunchKernelGGL(kern, dim3(tiles, Y, (ka + apb - 1) / apb), dim3(NT_A), 0, s_, (const c32*)Ty_,
                              (const c32*)Tyn_, (const c32*)FI_, (const c32*)FIn_, Q_, tw_.f32(L), Y, Xh, nz, ka, apb);
         };
-        go(k_passA<L, TW, true>, 1);
-        if (Xh > TW) go(k_passA<L, TW, false>, Xh / TW - 1);
+        go(std::true_type{}, 1);
+        if (Xh > TW) go(std::false_type{}, Xh / TW - 1);
       } else {
         throw Error(ERR_UNSUPPORTED, "pass A tile does not fit in LDS");
       }
