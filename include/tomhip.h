@@ -156,12 +156,16 @@ int tomhip_search_profile(tomhip_search* s, int enable, double* ms, int64_t* cou
  * launch every kernel eagerly (0). Results are identical. */
 int tomhip_search_set_graph(tomhip_search* s, int enable);
 /* Column-tile widths (8, 16 or 32; default 16) of the z-FFT pass and the
- * y-FFT pass: workgroup shape only, results are identical. No reference
+ * y-FFT pass; results are identical. Large batches of the common lengths run
+ * two kernels without tiles instead, where these have no effect, except that
+ * at Z = 256 a z tile other than 16 selects the separate passes. No reference
  * counterpart; set by the autotuner. */
 int tomhip_search_set_tiles(tomhip_search* s, int tile_z, int tile_y);
 /* Run the y-FFT and c2r/max passes over z-chunks of this many planes (0 =
  * whole volume), so the c2r pass reads the y pass's output back from the
- * memory-side cache. Results are identical. No reference counterpart. */
+ * memory-side cache. Any chunk, Z among them, selects the separate passes, 0
+ * leaves the choice to the search (above). Results are identical. No reference
+ * counterpart. */
 int tomhip_search_set_zchunk(tomhip_search* s, int planes);
 void tomhip_search_destroy(tomhip_search* s);
 

@@ -436,11 +436,14 @@ class SearchPlan:
         return sc, an, pos
 
     def set_tiles(self, tile_z: int = 16, tile_y: int = 16):
-        """Column-tile widths of the z- and y-FFT passes (8, 16 or 32)."""
+        """Column-tile widths of the z- and y-FFT passes (8, 16 or 32). Without
+        effect where a batch runs the two-kernel inverse, which a z tile other
+        than 16 turns off at Z = 256."""
         self.ctx.check(self.ctx.lib.tomhip_search_set_tiles(self.h, int(tile_z), int(tile_y)))
 
     def set_zchunk(self, planes: int = 0):
-        """Run the y-FFT and c2r/max passes over z-chunks (0 = whole volume)."""
+        """Run the y-FFT and c2r/max passes over z-chunks (0 = whole volume);
+        any chunk turns the two-kernel inverse of large batches off."""
         self.ctx.check(self.ctx.lib.tomhip_search_set_zchunk(self.h, int(planes)))
 
     def set_graph(self, enable: bool):

@@ -4,7 +4,11 @@ template-spectrum and Q tiles and the register-resident max of the c2r pass)
 the column-tile widths of the z- and y-FFT passes and the z-chunking of the
 last two passes, by timing a few launch groups of each candidate through
 hipGraph replay as in production. The search is staged: batch first (default
-tiles), then the z tile, then the y tile, then the chunk.
+tiles), then the z tile, then the y tile, then the chunk. Large batches of the
+common lengths run two kernels that have no tiles (the search's y transform is
+not launched by itself); a tile stage is left out there, except the z tile's at
+Z = 256, where a width other than 16 selects the separate passes, as a chunk
+does.
 
 None of these change the mathematics (each voxel keeps the first strictly
 better orientation in list order, whatever the grouping); the FP32 sums may
@@ -12,8 +16,8 @@ round differently by a few ulp, which can flip the best orientation only in
 near-ties. `tune_search` compares every candidate's maps with the first and
 fails loudly when a score differs by more than 1e-6 or when more than 1e-5 of
 the voxels change their best orientation.
-Results are cached per (device, volume shape, template shape) in
-$TOM_AMD_CACHE (default ~/.cache/tom_amd/autotune.json).
+Results are cached per (set of kernels, device, volume shape, template shape)
+in $TOM_AMD_CACHE (default ~/.cache/tom_amd/autotune.json).
 """
 from __future__ import annotations
 
@@ -33,6 +37,9 @@ ZCHUNKS = (0, 64, 32)
 SCORE_ULP_TOL = 1e-6
 # largest fraction of voxels whose best orientation may flip (near-ties)
 ANGLE_FLIP_FRAC = 1e-5
+# of the kernels that the settings choose between: a result of another set is
+# no result (a tile or a chunk may select passes that are now the slower ones)
+KERNELS = "k2"
 
 
 def _cache_path():
@@ -43,7 +50,7 @@ def _cache_path():
 def _key(volume_dims, template_shape):
     import torch
     name = torch.cuda.get_device_name(0) if torch.cuda.is_available() else "cpu"
-    return f"{name}|{tuple(int(d) for d in volume_dims)}|{tuple(int(d) for d in template_shape)}"
+    return f"{KERNELS}|{name}|{tuple(int(d) for d in volume_dims)}|{tuple(int(d) for d in template_shape)}"
 
 
 def tune_search(volume, tmpl, mask, W, mu_t, sig_t, angles, batches=BATCHES, tiles=TILES, zchunks=ZCHUNKS,
@@ -67,10 +74,14 @@ def tune_search(volume, tmpl, mask, W, mu_t, sig_t, angles, batches=BATCHES, til
             return dict(cache[key], cached=True)
     ang = np.asarray(angles, np.float32)[:max(batches) * groups]
     timing = {}
+    tiled = {}
     ref = []
 
+    def label(ka, tz, ty, zc):
+        return f"batch{ka}_z{tz}_y{ty}_c{zc}"
+
     def trial(ka, tz, ty, zc):
-        name = f"batch{ka}_z{tz}_y{ty}_c{zc}"
+        name = label(ka, tz, ty, zc)
         with api.SearchPlan(volume, tshape, mask, batch=ka) as p:
             try:
                 p.set_tiles(tz, ty)
@@ -78,6 +89,9 @@ def tune_search(volume, tmpl, mask, W, mu_t, sig_t, angles, batches=BATCHES, til
                 return None  # tile does not fit this volume
             p.set_zchunk(zc)
             p.set_template(tmpl, W, mu_t, sig_t)
+            p.profile(True)
+            p.run(ang[:ka], 0)
+            tiled[name] = bool(p.profile(False)[1][4])  # y passes of their own
             p.run(ang[:2 * ka], 0)  # capture + warm
             p.set_template(tmpl, W, mu_t, sig_t)
             torch.cuda.synchronize()
@@ -107,6 +121,9 @@ def tune_search(volume, tmpl, mask, W, mu_t, sig_t, angles, batches=BATCHES, til
     best = {"batch": 4, "tile_z": 16, "tile_y": 16, "zchunk": 0}
     for stage, values in (("batch", batches), ("tile_z", tiles), ("tile_y", tiles), ("zchunk", zchunks)):
         scores = {}
+        now = label(*(best[k] for k in ("batch", "tile_z", "tile_y", "zchunk")))
+        if not tiled.get(now, True) and (stage == "tile_y" or (stage == "tile_z" and int(vb.dims[2]) != 256)):
+            continue
         for v in values:
             cfg = dict(best, **{stage: v})
             ms = trial(cfg["batch"], cfg["tile_z"], cfg["tile_y"], cfg["zchunk"])
