@@ -240,8 +240,9 @@ void box_prepare(Twiddles& tw, int nx, int ny, int nz) {
   for (int L : {nx, ny, nz}) (void)line_list(tw, L);
 }
 
-void box_filter(Twiddles& tw, hipStream_t s, int count, float* t, c32* work, const float* wsh, const float* mask,
-                int nx, int ny, int nz) {
+// count up to 65,535: a grid dimension
+static void box_filter_slab(Twiddles& tw, hipStream_t s, int count, float* t, c32* work, const float* wsh,
+                            const float* mask, int nx, int ny, int nz) {
   const long n3 = (long)nx * ny * nz;
   const long lpv = (long)ny * nz;  // x lines per box
   const long XY = (long)nx * ny;
@@ -268,12 +269,11 @@ void box_filter(Twiddles& tw, hipStream_t s, int count, float* t, c32* work, con
     });
   }
   TOMHIP_CHECK(hipGetLastError());
-  for (int b = 0; b < count; b += 65535)
-    dispatch_box(nz, [&](auto Lc) {
-      constexpr int L = decltype(Lc)::value;
-      hipLaunchKernelGGL(k_box_z<L>, dim3((unsigned)((XY + 63) / 64), (unsigned)std::min(count - b, 65535)),
-                         dim3(64 * NW), 0, s, work + b * n3, wsh, (int)XY, line_list(tw, L));
-    });
+  dispatch_box(nz, [&](auto Lc) {
+    constexpr int L = decltype(Lc)::value;
+    hipLaunchKernelGGL(k_box_z<L>, dim3((unsigned)((XY + 63) / 64), (unsigned)count), dim3(64 * NW), 0, s, work, wsh,
+                       (int)XY, line_list(tw, L));
+  });
   TOMHIP_CHECK(hipGetLastError());
   if (plane) {
     dispatch_box(nx, [&](auto Lc) {
@@ -298,6 +298,13 @@ void box_filter(Twiddles& tw, hipStream_t s, int count, float* t, c32* work, con
                        (const c32*)work, t, mask, lpv, (float)(1.0 / (double)n3), tw.f32(L));
   });
   TOMHIP_CHECK(hipGetLastError());
+}
+
+void box_filter(Twiddles& tw, hipStream_t s, int count, float* t, c32* work, const float* wsh, const float* mask,
+                int nx, int ny, int nz) {
+  const long n3 = (long)nx * ny * nz;
+  for (int b = 0; b < count; b += 65535)
+    box_filter_slab(tw, s, std::min(count - b, 65535), t + b * n3, work + b * n3, wsh, mask, nx, ny, nz);
 }
 
 }  // namespace tomhip
