@@ -422,13 +422,16 @@ __device__ __forceinline__ void class_stages(c32* buf, const c32* tw, int w, int
 // eight waves have 256 registers each for the maxima (72), the next angle's
 // inputs (64) and the 32 elements at work; 16 waves of 128 registers spill
 // (2.35 ms). An angle has three exchanges through LDS and four barriers.
-template <int XH, int Y>
+// GROUPS: the angles in groups of apb (grid.y), each one's maxima for the merge
+// to pv and pi (a kernel of its own: with the choice made at run time the
+// undivided batch takes 1.63 for 1.61 ms here, 204 for 196 us at 256x256x128).
+template <int XH, int Y, bool GROUPS>
 __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __restrict__ Q, float* __restrict__ maxc,
                                                                 int32_t* __restrict__ argm,
                                                                 const c32* tw, int Z, int ka, int first_index,
                                                                 const long* desc, int apb, float* __restrict__ pv,
                                                                 uint8_t* __restrict__ pi, long n) {
-  const int a0 = blockIdx.y * apb, a1 = min(a0 + apb, ka);
+  const int a0 = GROUPS ? blockIdx.y * apb : 0, a1 = GROUPS ? min(a0 + apb, ka) : ka;
   if (desc) first_index = (int)(desc[1] + desc[0] * ka);
   using I1 = ClassStage<XH, Y, 1>;
   constexpr int NW = waves_bc(XH), NT_ = 64 * NW, R0 = I1::R0, Lp = I1::Lp, ZB = I1::ZB;
@@ -470,7 +473,7 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
     }
     return ((I1::NQ * NCH1) % NW == 0 || k < I1::NQ * NCH1) && zl < (PAIR ? nzb / 2 : nzb);
   };
-  const c32* qp = Q + a0 * Z * SU + (long)z0 * 2 * SU + (long)rc * Lp * XH * 2 + bit;
+  const c32* qp = Q + (GROUPS ? a0 * Z * SU : 0) + (long)z0 * 2 * SU + (long)rc * Lp * XH * 2 + bit;
   // quarter part of the loads of one angle (all of them: part < 0)
   auto fetch = [&](const c32* qa, int part, int w, int lane) {
 #pragma unroll
@@ -499,7 +502,7 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
 #pragma unroll
   for (int p = 0; p < NI; ++p) ix[p] = iy[p] = 0u;
 #pragma unroll
-  for (int k = 0; k < EPT; ++k) bx[k] = by[k] = -INFINITY;
+  for (int k = 0; k < EPT; ++k) bx[k] = by[k] = GROUPS ? -INFINITY : 0.f;
   fetch(qp, -1, w_, lane_);
   for (int a = a0; a < a1; ++a) {
     const int lane = fresh(lane_), w = fresh_uniform(w_);
@@ -607,9 +610,8 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
         });
     ahead(a, 3, w, lane);
   }
-  const int first = pv ? 0 : first_index;
-  // the batch's maximum against the resident maps (a group's, for
-  // merge_groups, to pv and pi), a quarter of every line at
+  const int first = GROUPS ? 0 : first_index;
+  // the batch's maximum against the resident maps, a quarter of every line at
   // a time through LDS so that the maps are read and written in rows
   constexpr int KC = EPT / 4, NS = NW * KC, FP = NS + 1;
   static_assert(EPT % 4 == 0 && 64 * FP * 2 <= 64 * P, "staging area");
@@ -632,7 +634,7 @@ __global__ __launch_bounds__(64 * waves_bc(XH)) void k_fused_bc(const c32* __res
       const long vx = (line * XH + r * NS + e) * 2;
       const float2 nv = sval[l * FP + e];
       const int2 ni = sidx[l * FP + e];
-      if (pv) {
+      if constexpr (GROUPS) {
         *reinterpret_cast<float2*>(pv + blockIdx.y * n + vx) = nv;
         *reinterpret_cast<uchar2*>(pi + blockIdx.y * n + vx) = make_uchar2(ni.x, ni.y);
         continue;
@@ -793,9 +795,15 @@ void fused_bc(Twiddles& tw, hipStream_t s, const c32* Q, float* maxc, int32_t* a
   dispatch_x(X / 2, [&](auto Xc) {
     dispatch_y(Y, [&](auto Yc) {
       constexpr int XH = decltype(Xc)::value, YL = decltype(Yc)::value;
-      hipLaunchKernelGGL((k_fused_bc<XH, YL>), dim3((unsigned)bc_blocks(YL, Z), (unsigned)((ka + apb - 1) / apb)),
-                         dim3(64 * waves_bc(XH)), 0, s, Q, maxc, argm, bc_list(tw, X, YL), Z, ka, first_index,
-                         desc, apb, pv, pi, (long)X * Y * Z);
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)bc_blocks(YL, Z), (unsigned)((ka + apb - 1) / apb)),
+                           dim3(64 * waves_bc(XH)), 0, s, Q, maxc, argm, bc_list(tw, X, YL), Z, ka, first_index, desc,
+                           apb, pv, pi, (long)X * Y * Z);
+      };
+      if (pv)
+        go(k_fused_bc<XH, YL, true>);
+      else
+        go(k_fused_bc<XH, YL, false>);
     });
   });
   TOMHIP_CHECK(hipGetLastError());

@@ -10,7 +10,8 @@ namespace tomhip {
 
 // Channels-last implicit-GEMM 3D convolution (zero padding, stride 1).
 // X: bf16 [D][H][W][xs], channels [xo, xo + Cin); Wt: bf16 [taps][Cout][Cin]
-// (taps 27 = 3x3x3 with tap t = 9(dz+1) + 3(dy+1) + (dx+1), or 1);
+// (taps 27 = 3x3x3 with tap t = 9(dz+1) + 3(dy+1) + (dx+1), or 1, the head's
+// forward and its data gradient);
 // output Yb (bf16, stride ys, offset yo) and/or Yf (f32 [V][Cout]).
 // Wm: the same weights in MFMA fragment order (conv_fragments), read
 // instead of Wt when taps == 27.
