@@ -249,11 +249,11 @@ __global__ __launch_bounds__(NTT) void k_tmpl_fwd_y(const c32* Tx, c32* Ty, c32*
     if (uy >= ny) return mk(0.f, 0.f);
     return (c < TW) ? src[(long)uy * XP + c] : srn[(long)uy * XP];
   };
-  c32* dst = Ty + ((long)a * nz + uz) * Y * Xh;
+  c32* dst = Ty + ((long)a * nz + uz) * Y * Xh + (TILED ? 0 : tile * TW);
   c32* dn = Tyn + ((long)a * nz + uz) * Y;
   auto st = [&](int, int, int c, int ky, c32 v) {
     if (c < TW)
-      dst[TILED ? fused_ty_index(Y, ky, tile * TW + c) : (long)ky * Xh + tile * TW + c] = v;
+      dst[TILED ? fused_ty_index(Y, ky, tile * TW + c) : (long)ky * Xh + c] = v;
     else
       dn[ky] = v;
   };
@@ -1365,7 +1365,7 @@ static int angle_groups(int blocks, int ka, int per_cu) {
     if ((ka + apb - 1) / apb != g) continue;
     const int n = (blocks * g + 255) / 256, rem = n % per_cu;
     const double t = (n / per_cu * (per_cu + 1) + (rem ? rem + 1 : 0)) * (apb + 0.7);
-    if (g == 1 || t < 0.97 * least) {
+    if (g == 1 || t < 0.98 * least) {
       best = g;
       least = t;
     }
