@@ -544,7 +544,7 @@ def tom_os3_angleList(start, end, increment, dedup: bool = True) -> np.ndarray:
 
 def subtomo_score_batch(boxes, particles, particle_box, wedge_semi_deg, angles, ctx: Optional[Context] = None):
     """Batched local angular search of subtomograms (tom_av3_corr3d 'peak' /
-    corr3d_batch semantics, one persistent launch).
+    corr3d_batch semantics, one call).
 
     boxes: list of dicts {"template": (B,B,B), "mask": (B,B,B), "mask_cc":
     (B,B,B) or None, "wedge_ref": semi-angle of the template's missing wedge in
