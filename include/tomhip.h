@@ -213,7 +213,7 @@ int tomhip_os3_bestpeak_f32(tomhip_ctx* ctx, const int64_t N[3], int rule, int32
 
 /* ---------------------------------------------------------------- subtomogram scoring */
 /* Batched, per-particle local angular search with per-particle wedges, in one
- * persistent launch: the 'peak' mode of tom_mex_corr3d
+ * call: the 'peak' mode of tom_mex_corr3d
  * (Oscar3/c++Picker/src/mex/tom_mex_corr3d.cpp:53-806 -> tom::corr3d_batch,
  * src/tom/corr/corr.cpp:969-1400, CorrelationHandlerPeaks
  * src/tom/corr/correlation_handler.cpp:96-120; MATLAB av3_new/tom_av3_corr3d.m)

@@ -758,13 +758,13 @@ bool fused_supported(int X, int Y, int Z, int ka) {
   if (8L * ka * Z * Y * (X / 2) < (192L << 20)) return false;
   if (!(dispatch_z(Z, [](auto) {}) && dispatch_x(X / 2, [](auto) {}) && dispatch_y(Y, [](auto) {}))) return false;
   // 1,402 batches of all these lengths, 192 MB to 3 GB, whole runs, separate
-  // passes over fused kernels: Z = 32 and 64 1.03 to 1.46; from 128 on 0.80 to
-  // 1.54, slower with the fused ones at Z = 192 (one block of 8 waves a CU),
-  // with few angles to a block of fused_a, and with the last round of
-  // fused_bc's blocks nearly empty. The sum below is a fit to the difference,
-  // in ns per 10^6 bytes of Q (the separate passes take 1,000 to 1,400), and
-  // where it is positive the ratio is 0.93 to 1.54, below 0.98 in 31 of 910;
-  // where it is not, 0.80 to 1.15 in 255.
+  // passes over fused kernels: Z = 32 and 64 1.03 to 1.46; from 128 on 0.81 to
+  // 1.57, slower with the fused ones at Z = 192 (one block of 8 waves a CU),
+  // with few angles to a block of fused_a, and where the last of fused_bc's
+  // blocks leave most CUs empty. The sum below is a fit to the difference, in ns
+  // per 10^6 bytes of Q (the separate passes take 1,000 to 1,400). Where it is
+  // positive the ratio is 0.94 to 1.57, below 0.98 in 28 of 910; where it is
+  // not, 0.81 to 1.14 in 255.
   if (Z < 128) return true;
   const int nb = bc_blocks(Y, Z) * fused_bc_groups(X, Y, Z, ka);
   const int y = (Y & (Y - 1)) == 0 ? 250 : Y < 200 ? 320 : 390;  // fused_bc's own time
